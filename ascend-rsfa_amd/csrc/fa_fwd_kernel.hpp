@@ -625,14 +625,25 @@ fa_fwd_kernel(FwdParams p) {
     constexpr bool PAIRS = CAUSAL && MODE == MODE_FUSED;
     const Queue qu = make_queue<PAIRS>(p);
     uint32_t* const ctr = p.ticket ? p.ticket + 16 * qu.x : nullptr;
-    int t;
-    if (ctr) {
-        if (tid == 0) *tslot = (int)atomicAdd(ctr, 1u);
-        __syncthreads();
-        t = task_of_ticket(qu, *tslot);
-        if constexpr (QPF) __syncthreads();  // read before the first task writes the slot again
-    } else {
-        t = task_of_ticket(qu, qu.rank);
+    // A workgroup's first ticket is its rank, and the queue's counter hands out
+    // the tickets from nwg on.  (Drawn like the others, the first one opened
+    // every launch with the round trip of a device-scope atomic, about 4k
+    // cycles: B=2 H=8 S=1024 D=128 causal 29.1 -> 27.7 us, B=1 H=8 S=8192 172.7
+    // -> 170.2, B=32 H=8 S=2048 D=32 230 -> 223.)  Except where pairs run in
+    // lockstep rounds and no task loads the next one's Q early: started in one
+    // burst those workgroups miss L2 on the same tiles together (B=4 H=16 S=8192
+    // D=64 566 us drawn, 570 by rank; B=64 H=8 S=1024 D=256 364 and 367; at
+    // D = 128, B=128 H=8 S=2048, 1241 and 1236).
+    constexpr bool DRAW_FIRST = PAIRS && D != 128;
+    const int base = DRAW_FIRST ? 0 : qu.nwg;
+    int t = task_of_ticket(qu, qu.rank);
+    if constexpr (DRAW_FIRST) {
+        if (ctr) {
+            if (tid == 0) *tslot = (int)atomicAdd(ctr, 1u);
+            __syncthreads();
+            t = task_of_ticket(qu, *tslot);
+            if constexpr (QPF) __syncthreads();  // read before the first task writes the slot again
+        }
     }
     bool qready = false;  // QPF: the previous task loaded this task's Q into the Q buffer
 
@@ -1344,7 +1355,7 @@ fa_fwd_kernel(FwdParams p) {
                     // tiles and the next one a whole query block, its Q is loaded
                     // in the phases X_{j0+2} and X_{j0+3}
                     const int tn = pair_continues(p, qu, t) ? t + 1
-                                   : task_of_ticket(qu, ctr ? __builtin_amdgcn_readfirstlane(*tslot)
+                                   : task_of_ticket(qu, ctr ? base + __builtin_amdgcn_readfirstlane(*tslot)
                                                             : ticket_of_task(qu, t) + qu.nwg);
                     if (ctr) t_next = tn;
                     if (tn < qu.ntask && jpp - j0 >= 4) {
@@ -1606,7 +1617,7 @@ fa_fwd_kernel(FwdParams p) {
             } else {
                 if (tid == 0) *tslot = nxt;
                 __syncthreads();
-                t = task_of_ticket(qu, *tslot);
+                t = task_of_ticket(qu, base + *tslot);
                 if constexpr (QPF) __syncthreads();  // read before the next task writes the slot
             }
         } else {
@@ -1617,9 +1628,9 @@ fa_fwd_kernel(FwdParams p) {
     }
 
     // The workgroup holding the last ticket handed out by its queue returns the
-    // counter to zero for the next launch on this stream: every workgroup of
-    // the queue draws exactly one ticket >= ntask, so that ticket is
-    // ntask + nwg - 1.
+    // counter to zero for the next launch on this stream.  Serving a ticket draws
+    // one more, and so does a first ticket that was drawn: either way the last
+    // ticket is nwg - 1 past the tickets to serve.
     if (ctr && tid == 0 && ticket_of_task(qu, t) == ticket_of_task(qu, qu.ntask) + qu.nwg - 1) atomicExch(ctr, 0u);
 }
 

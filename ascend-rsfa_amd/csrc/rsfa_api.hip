@@ -178,6 +178,17 @@ int32_t use_pairs(int64_t num_heads, int32_t nmb, int64_t grid, int32_t nq) {
     return paired <= 1.03 * single ? 1 : 0;
 }
 
+// Whether a launch hands out more tickets than the workgroups' first ones (each
+// serves its rank in its queue without drawing).  Where every queue has a
+// workgroup per ticket, the counters are left out: the atomic that draws a
+// ticket past the end is then no part of a task (one 64-key tile on 8 heads
+// 5.7 -> 5.5 us, four 197-key ones on 128 heads 10.0 -> 9.4).
+bool queue_needed(const FwdParams& p, int64_t grid) {
+    const int64_t heads = (p.num_heads + p.nq - 1) / p.nq;  // of the fullest queue
+    const int64_t tickets = heads * (p.pairs ? (p.nmb + 1) / 2 : p.nmb);
+    return tickets > grid / p.nq;
+}
+
 // Position of an instantiation in the kernel lists (a fixed-size cache index).
 int kernel_index(const KernelEntry& e) {
     int base = 0;
@@ -535,13 +546,6 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
         p.acc = p.state + 2 * (int64_t)p.num_tasks * bm;
     }
 
-    const bool dynamic = !(a->flags & RSFA_FLAG_STATIC_SCHEDULE) && (tickets_given || dynamic_schedule_allowed(stream));
-    if (dynamic && tickets_given) {
-        // caller-placed counters start each call at zero (a launch leaves
-        // them at zero, but the caller's buffer may hold anything)
-        hipLaunchKernelGGL(clear_words, dim3(1), dim3(64), 0, (hipStream_t)stream, tickets, kSlotWords);
-        if (hipGetLastError() != hipSuccess) return RSFA_E_LAUNCH;
-    }
     const int modes[2] = {split ? MODE_PREFIX : MODE_FUSED, MODE_DIAG};
     const int launches = split ? 2 : 1;
     for (int li = 0; li < launches; ++li) {
@@ -556,7 +560,21 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
         p.pairs = causal && modes[li] == MODE_FUSED && !(a->flags & RSFA_FLAG_SINGLE_BLOCKS)
                       ? use_pairs(p.num_heads, p.nmb, grid, p.nq)
                       : 0;
-        p.ticket = !dynamic ? nullptr : tickets_given ? tickets : stream_ticket(ds, stream);
+        p.ticket = nullptr;
+        if (!(a->flags & RSFA_FLAG_STATIC_SCHEDULE) && queue_needed(p, grid)) {
+            if (!tickets_given) {
+                if (dynamic_schedule_allowed(stream)) p.ticket = stream_ticket(ds, stream);
+            } else {
+                p.ticket = tickets;
+                if (li == 0) {
+                    // caller-placed counters start each call at zero (a launch
+                    // leaves them at zero, but the caller's buffer may hold
+                    // anything)
+                    hipLaunchKernelGGL(clear_words, dim3(1), dim3(64), 0, (hipStream_t)stream, tickets, kSlotWords);
+                    if (hipGetLastError() != hipSuccess) return RSFA_E_LAUNCH;
+                }
+            }
+        }
         void* args[] = {&p};
         if (hipLaunchKernel(k->fn, dim3((unsigned)grid), dim3((unsigned)(k->nw * 64)), args, 0,
                             (hipStream_t)stream) != hipSuccess)
