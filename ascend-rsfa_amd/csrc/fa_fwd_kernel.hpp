@@ -36,11 +36,17 @@
 //   (211, 456); the row sum adds the rounded values (v_dot2 with ones).
 //
 // LDS layout of one K or V tile (BN rows x DP cols, 2-byte elements)
-//   rows are grouped in blocks of 16; inside a block the 16-byte chunk c of row
-//   r sits at  c*256 + ((r%16) ^ (4*(c%4)))*16.  Each 256-byte chunk plane holds
-//   16 rows, so a half-wave's 16-byte K reads and the 16-lane groups of the
-//   transposing V reads both touch 64 distinct banks, and one wave's direct
-//   load instruction fills 1 KB of consecutive LDS.
+//   rows are grouped in blocks of 16, and a block's columns in planes of 32
+//   (1 KB: 16 rows x 64 bytes, one wave's direct load); row r of a plane keeps
+//   its 16-byte chunk c at column c ^ row_swz(r), so the 16-lane groups of the
+//   K reads (16 rows, one chunk) and the 32-lane halves of the transposing V
+//   reads (4 rows, four chunks) touch 64 distinct banks.  Four consecutive lanes
+//   of a direct load thus fetch 64 consecutive bytes: the CU's address unit
+//   takes such quads whole, 41 bytes per clock and CU with all CUs loading from
+//   L2 (61 with one CU per XCD), while lanes that walk down the rows, 16 bytes
+//   each (planes of one chunk column instead), pass one per clock: 16 (B=2 H=8
+//   S=1024 D=128 causal 27.8 us so, 26.3 in quads; B=128 H=8 S=2048 causal 1234
+//   and 1208, non-causal 2013 and 1990, with a float8 V at B=32 393 and 384).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -59,6 +65,9 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
+
+// Column swizzle of row r (mod 16) of a plane: rows 4 apart share banks.
+__device__ __forceinline__ int row_swz(int r) { return 2 * ((r >> 2) & 1) + ((r >> 3) & 1); }
 
 // How far (in log2 units) the running row max may lag the true max before the
 // accumulator is rescaled.  P = 2^(s*c - m) stays <= 2^15, inside the normal
@@ -513,7 +522,7 @@ fa_fwd_kernel(FwdParams p) {
     // K (A operand of S^T): row l32 (+32 per sub-tile), chunk 2s+hh.
     uint32_t koff[2];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) koff[e] = (l32 >> 4) * BLK + hh * 256 + ((l16 ^ (8 * e + 4 * hh)) * 16);
+    for (int e = 0; e < 2; ++e) koff[e] = (l32 >> 4) * BLK + l16 * 64 + ((2 * e + hh) ^ row_swz(l16)) * 16;
     // At D = 256 (O^T and Q^T hold 192 of the 256 VGPRs) values the compiler
     // hoists out of the task loop are spilled, and each reload from scratch
     // makes it wait for every load in flight (vmcnt(0)): at a task's start the
@@ -532,10 +541,11 @@ fa_fwd_kernel(FwdParams p) {
     // its 16 head dims; the hardware hands lane j column j of the 4 rows.
     const int vg = (lane >> 4) & 1;
     const int vcc = 2 * vg + ((l16 >> 1) & 1);
+    auto vrow = [&](int u) { return 8 * u + 4 * hh + (l16 >> 2); };
     uint32_t voff[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
-        voff[u] = vcc * 256 + (((8 * u + 4 * hh + (l16 >> 2)) ^ (4 * vcc)) * 16) + 8 * (l16 & 1);
+        voff[u] = vrow(u) * 64 + (vcc ^ row_swz(vrow(u))) * 16 + 8 * (l16 & 1);
     // V8 (ds_read_b64_tr_b8): in a 16-lane group lanes 2r and 2r+1 address
     // bytes 0-7 and 8-15 of row r of eight rows, and the hardware hands lane j
     // column j of the eight rows.  The read of 16-key group q' (keys 16q'.. of
@@ -575,11 +585,11 @@ fa_fwd_kernel(FwdParams p) {
         }
     };
 
-    // Loader: in every 1-KB slice lane i fills chunk 4*cg + i/16 of the 16-row
-    // block's row (i%16) ^ 4*((i/16)%4), so its global offset inside the block
-    // is the same for every slice.
-    const int ld_rib = l16 ^ (4 * ((lane >> 4) & 3));
-    const int ld_chl = lane >> 4;
+    // Loader: slice w is plane cg of 16-row block blk; in every slice lane i fills
+    // column i%4 of row i/4, with that row's chunk 4*cg + (i%4 ^ row_swz), so its
+    // global offset inside the block is the same for every slice.
+    const int ld_rib = lane >> 2;
+    const int ld_chl = (lane & 3) ^ row_swz(ld_rib);
     // Byte offsets of this wave's slices (slice w = sl*NW + wave) from the first
     // row of a whole tile, for K and V; the tile loop only adds a uniform base.
     constexpr int NSL = (NINST + NW - 1) / NW;
@@ -849,7 +859,7 @@ fa_fwd_kernel(FwdParams p) {
             i32x4 r[KST];
             static_for<KST>([&](auto sc) {
                 constexpr int s = decltype(sc)::value;
-                r[s] = lds_read_b128<s * 512>((s & 1) ? qa1 : qa0);
+                r[s] = lds_read_b128<(s >> 1) * 1024>((s & 1) ? qa1 : qa0);
             });
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
@@ -963,7 +973,7 @@ fa_fwd_kernel(FwdParams p) {
                 auto issue = [&](auto ic) {
                     constexpr int i = decltype(ic)::value;
                     constexpr int ss = i / NKT, kt = i % NKT;
-                    ring[i % NB] = lds_read_b128<kt * 2 * BLK + ss * 512>((ss & 1) ? kb1 : kb0);
+                    ring[i % NB] = lds_read_b128<kt * 2 * BLK + (ss >> 1) * 1024>((ss & 1) ? kb1 : kb0);
                 };
                 static_for<PF>(issue);
                 static_for<NM>([&](auto ic) {
@@ -981,7 +991,7 @@ fa_fwd_kernel(FwdParams p) {
 #pragma unroll
                     for (int kt = 0; kt < NKT; ++kt) {
                         if (kt < nkt_act) {
-                            const x8 a = *(const RSFA_LDS x8*)(kt_lds + koff[s & 1] + kt * 2 * BLK + s * 512);
+                            const x8 a = *(const RSFA_LDS x8*)(kt_lds + koff[s & 1] + kt * 2 * BLK + (s >> 1) * 1024);
                             sacc[kt] = T::mfma(a, qf[s], s == 0 ? zero : sacc[kt]);
                         }
                     }
@@ -1235,7 +1245,7 @@ fa_fwd_kernel(FwdParams p) {
                         }
                     } else {
                         constexpr int i = m - NPV, ss = i / NKT, kt = i % NKT;
-                        kr[i % XNB] = lds_read_b128<kt * 2 * BLK + ss * 512>(xa[2 + (ss & 1)]);
+                        kr[i % XNB] = lds_read_b128<kt * 2 * BLK + (ss >> 1) * 1024>(xa[2 + (ss & 1)]);
                     }
                 };
                 // X phase of PV(tv) and, when M > NPV, QK(tv + 1); with tl >= 0 it
