@@ -496,6 +496,15 @@ fa_fwd_kernel(FwdParams p) {
     constexpr bool QPF = uses_q_buffer(D, BN, NW, CAUSAL, MODE);
     static_assert(!QPF || (NBUF == 3 && NBUF * BUF + QTILE <= 160 * 1024), "Q buffer past the LDS");
 
+    // Q loaded into registers in quads and transposed through a part of the last
+    // K/V buffer, whose first loads go out in the first MFMA phase or later: a
+    // fragment's own load takes the address unit one clock per lane (B=2 H=8
+    // S=1024 D=128 causal 26.3 -> 25.6 us, B=1 H=8 S=2048 D=256 70.7 -> 69.8,
+    // B=64 H=8 S=1024 D=256 545 -> 542).  The kernels with a Q buffer load few Q
+    // rows this way, and the code made their causal loop 1 % slower.
+    constexpr bool QQUAD = D >= 64 && !QPF;
+    static_assert(!QQUAD || NW * 2048 <= BUF, "the staging of Q past the last K/V buffer");
+
     __shared__ __attribute__((aligned(1024))) char smem_raw[NBUF * BUF + (QPF ? QTILE : 0)];
     RSFA_LDS char* const smem = (RSFA_LDS char*)smem_raw;
     const uint32_t smem_addr = (uint32_t)(uintptr_t)smem;
@@ -872,9 +881,36 @@ fa_fwd_kernel(FwdParams p) {
         if (QPF && qready) {
             read_q();
         } else if (!q_dma) {
-            const elem* const ql = q_lane();
+            if constexpr (QQUAD) {
+                // 1-KB loads of 16 rows x 64 bytes, four lanes to a row, turned
+                // into fragments through 2 KB of LDS of the wave's own
+                const int ln = fresh_lane();
+                const int rr = m0 + wave * 32 + (ln >> 2), cc = (ln & 3) * 8;
+                const elem* const q0 = qb + (int64_t)min(rr, n - 1) * p.q_sm + cc;
+                const elem* const q1 = qb + (int64_t)min(rr + 16, n - 1) * p.q_sm + cc;
+                x8 r[KST];
 #pragma unroll
-            for (int s = 0; s < KST; ++s) qf[s] = *(const x8*)(ql + 16 * s);
+                for (int s = 0; s < KST / 2; ++s) {
+                    r[2 * s] = *(const x8*)(q0 + 32 * s);
+                    r[2 * s + 1] = *(const x8*)(q1 + 32 * s);
+                }
+                RSFA_LDS char* const qs = smem + (NBUF - 1) * BUF + wave * 2048;
+                const int wo = (ln >> 2) * 64 + ((ln & 3) ^ row_swz(ln >> 2)) * 16;
+                const int r32 = ln & 31, r16 = ln & 15;
+#pragma unroll
+                for (int s = 0; s < KST / 2; ++s) {
+                    *(RSFA_LDS x8*)(qs + wo) = r[2 * s];
+                    *(RSFA_LDS x8*)(qs + 1024 + wo) = r[2 * s + 1];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        qf[2 * s + e] = *(const RSFA_LDS x8*)(qs + (r32 >> 4) * 1024 + r16 * 64 +
+                                                              ((2 * e + ((ln >> 5) & 1)) ^ row_swz(r16)) * 16);
+                }
+            } else {
+                const elem* const ql = q_lane();
+#pragma unroll
+                for (int s = 0; s < KST; ++s) qf[s] = *(const x8*)(ql + 16 * s);
+            }
             // Q has arrived here as far as the compiler knows (the tile loops
             // wait for the first tile's loads, issued before Q's, anyway):
             // without this it would wait for Q, i.e. for the newest direct
