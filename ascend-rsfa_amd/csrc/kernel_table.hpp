@@ -44,6 +44,10 @@ KernelList kernels_d256();
     {DTYPE, D, BN, NW, 1, MODE_DIAG, OCC, 0, (const void*)&fa_fwd_kernel<T, D, BN, NW, true, MODE_DIAG, OCC>, \
      32 * NW}
 
+// The same, non-causal only.
+#define RSFA_TILE_NONCAUSAL(T, DTYPE, D, BN, NW, OCC)                                                \
+    {DTYPE, D, BN, NW, 0, MODE_FUSED, OCC, uses_pingpong(D, BN, NW, false, MODE_FUSED),                   \
+     (const void*)&fa_fwd_kernel<T, D, BN, NW, false, MODE_FUSED, OCC>, 32 * NW}
 
 #define RSFA_DEFINE_KERNEL_LIST(NAME, ...)                                   \
     namespace rsfa {                                                         \

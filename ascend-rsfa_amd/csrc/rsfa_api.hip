@@ -266,9 +266,13 @@ TileCost tile_cost(const KernelEntry& e, int64_t z, int64_t h, int64_t n, int nu
     // every CU, but no shorter than the longest task, whose waves each share
     // a SIMD with waves_per_simd - 1 others.
     double work = 0.0, longest = 0.0;
+    // task setup / epilogue; the wait for the first tile, of the few a short
+    // row has, decides between the 64- and the 128-key tiles of head dims 16
+    // and 32 (B=32 H=16 S=333 D=32: 23.1 and 24.4 us)
+    const double setup = 600.0 + (e.d <= 32 ? 16.0 * e.bn : 0.0);
     for (int64_t mb = 0; mb < nmb; ++mb) {
         const int64_t tiles = e.causal ? std::min<int64_t>(tiles_full, ((mb + 1) * bm + e.bn - 1) / e.bn) : tiles_full;
-        const double c = tiles * step + 600.0;  // + task setup / epilogue
+        const double c = tiles * step + setup;
         work += c * e.nw;
         longest = std::max(longest, c * waves_per_simd);
     }
