@@ -1,5 +1,5 @@
 // Instantiations of the forward kernel for head dim 128 (fp16, bf16, and fp16 with a float8 e5m2 V).
-#include "fa_fwd_kernel.hpp"
+#include "fa_fwd_keysplit.hpp"
 #include "kernel_table.hpp"
 
 using namespace rsfa;
@@ -12,5 +12,7 @@ using namespace rsfa;
 #endif
 
 // float8 V at head dim 128: V's bytes go into LDS as they are (TypeF16V8)
+#define RSFA_D128_KS(T, DTYPE) RSFA_KEYSPLIT_ENTRIES(T, DTYPE, 128, 128, 64, 64, 2), RSFA_KEYSPLIT_ENTRIES(T, DTYPE, 128, 128, 64, 32, 4)
+
 RSFA_DEFINE_KERNEL_LIST(kernels_d128, RSFA_D128_TILES(TypeF16, 0), RSFA_D128_TILES(TypeBF16, 1),
-                        RSFA_D128_TILES(TypeF16V8, 2))
+                        RSFA_D128_TILES(TypeF16V8, 2), RSFA_D128_KS(TypeF16, 0), RSFA_D128_KS(TypeBF16, 1))

@@ -1,5 +1,5 @@
 // Instantiations of the forward kernel for head dim 32 (fp16, bf16, and fp16 with a float8 e5m2 V).
-#include "fa_fwd_kernel.hpp"
+#include "fa_fwd_keysplit.hpp"
 #include "kernel_table.hpp"
 
 using namespace rsfa;
@@ -16,5 +16,7 @@ using namespace rsfa;
 #define RSFA_D32_TILES(T, DTYPE) RSFA_TILE_ENTRIES(T, DTYPE, 32, 64, 4, 4), RSFA_TILE_NONCAUSAL(T, DTYPE, 32, 128, 4, 3)
 #endif
 
+#define RSFA_D32_KS(T, DTYPE) RSFA_KEYSPLIT_ENTRIES(T, DTYPE, 32, 128, 64, 64, 4)
+
 RSFA_DEFINE_KERNEL_LIST(kernels_d32, RSFA_D32_TILES(TypeF16, 0), RSFA_D32_TILES(TypeBF16, 1),
-                        RSFA_D32_TILES(TypeF16V8, 2))
+                        RSFA_D32_TILES(TypeF16V8, 2), RSFA_D32_KS(TypeF16, 0), RSFA_D32_KS(TypeBF16, 1))

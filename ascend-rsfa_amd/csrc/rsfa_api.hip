@@ -51,8 +51,18 @@ void for_each_kernel(F&& f) {
 const KernelEntry* find_kernel(int dtype, int d, int bn, int bm, int causal, int mode) {
     const KernelEntry* hit = nullptr;
     for_each_kernel([&](const KernelEntry& e) {
-        if (e.dtype == dtype && e.d == d && e.bn == bn && e.bm == bm && e.causal == causal && e.mode == mode)
+        if (e.dtype == dtype && e.d == d && e.bn == bn && e.bm == bm && e.causal == causal && e.mode == mode && e.kg == 1)
             hit = &e;
+    });
+    return hit;
+}
+
+// Whether a tile has key-split variants.
+bool has_keysplit(const KernelEntry& tile) {
+    bool hit = false;
+    for_each_kernel([&](const KernelEntry& e) {
+        if (e.kg > 1 && e.dtype == tile.dtype && e.d == tile.d && e.causal == tile.causal && e.bm == tile.bm && e.bn == tile.bn)
+            hit = true;
     });
     return hit;
 }
@@ -285,12 +295,89 @@ TileCost tile_cost(const KernelEntry& e, int64_t z, int64_t h, int64_t n, int nu
     return tc;
 }
 
+// ---------------------------------------------------------------------------
+// Key-split variants (fa_fwd_keysplit.hpp).  A launch whose blocks are too few
+// or too unequal to fill the CUs runs shorter with smaller blocks whose keys
+// the waves of a workgroup share: twice as many tasks of half the length at
+// the same rate per CU (128 rows, two key groups), or four times as many (64
+// rows, four groups) that load K and V once per 64 rows.  Which one ends first
+// is read off this model: a task costs `task` + `step` per key tile (of all its
+// groups), in microseconds at the clock of a part-filled chip, the shared pair
+// where several workgroups of it sit on a CU; a launch takes as long as its
+// longest task, no less than its work spread over the workgroups, and, filled,
+// no less than 1.5 times that, since the board then runs at its power limit
+// (1.3 times for causal launches at head dim 128, whose short tasks leave the
+// matrix cores idle more: B*H = 32, S=2048 50 us in 256-row blocks, 43 split).
+// Fitted to kernel times of 593 shapes (2 to 256 heads, 64 to 8192 keys, fp16):
+// rms 7 to 10 % (head dim 32: 16 %).  (Head dim 256 has no variant: 128 rows
+// of its Q do not fit the buffers that are free at a task's start.)
+// ---------------------------------------------------------------------------
+struct LaunchCost {
+    int d, rows, bn, kg;  // rows and keys per step of a workgroup
+    int wgs;              // workgroups per CU
+    double task, step, task_shared, step_shared;
+};
+constexpr double LAUNCH_US = 4.0;
+constexpr LaunchCost launch_costs[] = {
+    {128, 256, 64, 1, 1, 3.00, 1.34, 0, 0},   {128, 128, 64, 1, 2, 2.04, 1.15, 3.44, 1.48},
+    {128, 128, 128, 2, 1, 2.90, 1.49, 0, 0},  {128, 64, 128, 4, 1, 2.85, 0.82, 0, 0},
+    {64, 256, 128, 1, 1, 3.03, 1.49, 0, 0},   {64, 128, 64, 1, 2, 1.07, 0.79, 2.31, 0.90},
+    {64, 128, 256, 2, 1, 2.92, 1.72, 0, 0},   {64, 64, 256, 4, 1, 2.36, 0.86, 0, 0},
+    {32, 128, 64, 1, 4, 0.23, 0.61, 1.25, 0.83}, {32, 128, 128, 1, 3, 0.23, 1.10, 1.25, 1.50},
+    {32, 64, 256, 4, 1, 2.06, 0.57, 0, 0},
+};
+
+// Predicted microseconds of a launch, or 0 where the model has no entry.
+double launch_us(const KernelEntry& e, int64_t heads, int64_t n, int num_cus) {
+    for (const LaunchCost& c : launch_costs) {
+        if (c.d != e.d || c.rows != e.rows || c.kg != e.kg || c.bn != e.keys * e.kg) continue;
+        const int64_t nmb = (n + c.rows - 1) / c.rows;
+        const int64_t tasks = heads * nmb;
+        const int64_t conc = std::max<int64_t>(1, std::min<int64_t>(c.wgs, (tasks + num_cus - 1) / num_cus));
+        const double task = conc > 1 ? c.task_shared : c.task, step = conc > 1 ? c.step_shared : c.step;
+        const int64_t slots = num_cus * conc;
+        const double longest = task + step * (double)((n + c.bn - 1) / c.bn);
+        double total = longest * (double)tasks, span;
+        if (e.causal) {
+            // block m has ceil((m + 1) rows / bn) steps: on average (nmb + 1) / 2
+            // blocks' worth and half a step of rounding up where a step is longer
+            const double rounding = c.bn > c.rows ? 0.5 * (1.0 - (double)c.rows / c.bn) : 0.0;
+            const double steps = std::min(0.5 * (double)(nmb + 1) * c.rows, (double)n) / c.bn + rounding;
+            total = (double)tasks * (task + step * std::max(1.0, steps));
+            span = std::max(longest, total / (double)std::min(slots, tasks));
+        } else {
+            span = (double)((tasks + slots - 1) / slots) * longest;
+        }
+        return LAUNCH_US + std::max(span, total / (double)slots * (e.causal && e.d == 128 ? 1.3 : 1.5));
+    }
+    return 0.0;
+}
+
+// The key-split variant that runs `base`'s shape at least a tenth shorter than
+// `base` (head dim 32, whose predictions are looser: 15 %), or `base`.  Over the
+// fitted shapes 268 run one, 1.15 to 1.22 times as fast in the geometric mean of
+// all; one is slower (B*H = 16, S=4096, D=32: 60.2 -> 63.9 us).
+const KernelEntry* keysplit_or(const KernelEntry* base, int64_t heads, int64_t n, int num_cus) {
+    const KernelEntry* best = base;
+    // (0 without an entry: no variant is shorter)
+    double limit = launch_us(*base, heads, n, num_cus) * (base->d == 32 ? 0.85 : 0.9);
+    for_each_kernel([&](const KernelEntry& e) {
+        if (e.kg == 1 || e.dtype != base->dtype || e.d != base->d || e.causal != base->causal) return;
+        const double us = launch_us(e, heads, n, num_cus);
+        if (us > 0.0 && us < limit) {
+            best = &e;
+            limit = us;
+        }
+    });
+    return best;
+}
+
 int choose_tiling(int64_t z, int64_t h, int64_t n, int64_t d, int causal, int dtype, int num_cus,
                   const KernelEntry** out) {
     const KernelEntry* best = nullptr;
     double best_cycles = 0.0;
     for_each_kernel([&](const KernelEntry& e) {
-        if (e.dtype != dtype || e.d != d || e.causal != (causal ? 1 : 0) || e.mode != MODE_FUSED) return;
+        if (e.dtype != dtype || e.d != d || e.causal != (causal ? 1 : 0) || e.mode != MODE_FUSED || e.kg > 1) return;
         const TileCost tc = tile_cost(e, z, h, n, num_cus);
         if (!tc.feasible) return;
         if (!best || tc.cycles < best_cycles - 1e-6 ||
@@ -300,7 +387,29 @@ int choose_tiling(int64_t z, int64_t h, int64_t n, int64_t d, int causal, int dt
         }
     });
     if (!best) return RSFA_E_TILE;
-    *out = best;
+    *out = keysplit_or(best, z * h, n, num_cus);
+    return RSFA_OK;
+}
+
+// choose_tiling's answer for a launch, kept per thread for the shapes last
+// asked for (the search takes longer than the rest of a launch).
+int choose_tiling_kept(int64_t z, int64_t h, int64_t n, int64_t d, int causal, int dtype, int num_cus,
+                       const KernelEntry** out) {
+    struct Kept {
+        int64_t zh, n;
+        int32_t d, causal, dtype, num_cus;
+        const KernelEntry* e;
+    };
+    static thread_local Kept kept[64] = {};
+    const int64_t zh = z * h;
+    Kept& k = kept[((uint64_t)(zh * 1000003 + n * 8191 + d * 31 + causal * 7 + dtype) * 0x9E3779B97F4A7C15ull) >> 58];
+    if (!(k.e && k.zh == zh && k.n == n && k.d == d && k.causal == causal && k.dtype == dtype && k.num_cus == num_cus)) {
+        const KernelEntry* e = nullptr;
+        const int st = choose_tiling(z, h, n, d, causal, dtype, num_cus, &e);
+        if (st != RSFA_OK) return st;
+        k = Kept{zh, n, (int32_t)d, causal, dtype, num_cus, e};
+    }
+    *out = k.e;
     return RSFA_OK;
 }
 
@@ -324,7 +433,7 @@ int resolve_exact(int64_t d, int causal, int dtype, int req_bm, int req_bn, cons
     const KernelEntry* best = nullptr;
     double best_dist = 0.0;
     for_each_kernel([&](const KernelEntry& e) {
-        if (e.dtype != dtype || e.d != d || e.causal != (causal ? 1 : 0) || e.mode != MODE_FUSED) return;
+        if (e.dtype != dtype || e.d != d || e.causal != (causal ? 1 : 0) || e.mode != MODE_FUSED || e.kg > 1) return;
         const double dist = std::fabs(std::log2((double)e.bm / req_bm)) + std::fabs(std::log2((double)e.bn / req_bn));
         if (!best || dist < best_dist - 1e-9 || (std::fabs(dist - best_dist) <= 1e-9 && e.bn > best->bn)) {
             best = &e;
@@ -356,7 +465,7 @@ int check_tensor(const void* ptr, const int64_t st[4], int mult = 8) {
 // row width) * 2 bytes must stay below 2^32, or the offsets would wrap.
 bool loader_offsets_fit(const KernelEntry& e, int64_t row_stride) {
     const int64_t dp = e.d < 32 ? 32 : e.d;
-    return ((int64_t)(e.bn - 1) * row_stride + dp) * 2 < (int64_t(1) << 32);
+    return ((int64_t)(e.keys - 1) * row_stride + dp) * 2 < (int64_t(1) << 32);
 }
 
 // Zeroes `words` 32-bit words (the no-allocation entry point's queue
@@ -449,16 +558,36 @@ uint64_t rsfa_split_workspace_bytes(int64_t z, int64_t h, int64_t n_ctx, int64_t
     return (uint64_t)(z * h * nmb * block_m) * (uint64_t)(2 + head_dim) * sizeof(float);
 }
 
-// The tile a launch runs: for a request (block_m, block_n), the nearest
-// compiled one, as the reference's BLOCK_M / BLOCK_N select its kernel's
-// tile; under RSFA_FLAG_TILE_HINT (unless RSFA_FLAG_EXACT_TILE) and without a
-// request, the tile search's choice for `num_cus` CUs (fwd_launch).
+// Whether a kernel's loaders can address the call's rows (below).
+static bool loaders_fit(const KernelEntry& e, const rsfa_fwd_args* a) {
+    const bool q_loader = e.kg > 1 || uses_q_buffer(e.d, e.bn, e.nw, e.causal != 0, e.mode);  // Q through LDS
+    return loader_offsets_fit(e, a->k_stride[2]) && loader_offsets_fit(e, a->v_stride[2]) &&
+           (!q_loader || loader_offsets_fit(e, a->q_stride[2]));
+}
+
+// The kernel a launch runs: for a request (block_m, block_n), that of the
+// nearest compiled tile, as the reference's BLOCK_M / BLOCK_N select its
+// kernel's tile; under RSFA_FLAG_TILE_HINT (unless RSFA_FLAG_EXACT_TILE) and
+// without a request, the tile search's choice for `num_cus` CUs.  Where that
+// choice is a key-split variant, a request for its tile runs it too; split
+// mode, and rows the variant cannot address, run the tile's plain kernel.
 static int launch_tile(const rsfa_fwd_args* a, int num_cus, const KernelEntry** e) {
-    const bool causal = a->causal != 0;
+    const int causal = a->causal != 0;
     const bool hint = (a->flags & RSFA_FLAG_TILE_HINT) && !(a->flags & RSFA_FLAG_EXACT_TILE);
-    if ((a->block_m != 0 || a->block_n != 0) && !hint)
-        return resolve_exact(a->head_dim, causal, a->dtype, a->block_m, a->block_n, e);
-    return choose_tiling(a->z, a->h, a->n_ctx, a->head_dim, causal, a->dtype, num_cus, e);
+    const bool requested = (a->block_m != 0 || a->block_n != 0) && !hint;
+    const bool split = causal && (a->flags & RSFA_FLAG_CAUSAL_SPLIT);
+    int st;
+    if (requested) {
+        if ((st = resolve_exact(a->head_dim, causal, a->dtype, a->block_m, a->block_n, e)) != RSFA_OK) return st;
+        if (split || !has_keysplit(**e)) return RSFA_OK;
+    }
+    const KernelEntry* best = nullptr;
+    if ((st = choose_tiling_kept(a->z, a->h, a->n_ctx, a->head_dim, causal, a->dtype, num_cus, &best)) != RSFA_OK)
+        return st;
+    if (best->kg > 1 && (split || !loaders_fit(*best, a)))
+        best = find_kernel(a->dtype, (int)a->head_dim, best->bn, best->bm, causal, MODE_FUSED);
+    if (!requested || (best->kg > 1 && best->bm == (*e)->bm && best->bn == (*e)->bn)) *e = best;
+    return RSFA_OK;
 }
 
 // Shared body of the launch entry points.  `ws` / `ws_bytes` is the
@@ -494,10 +623,7 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
     // <= Z*H*N_CTX rounded up to the largest BLOCK_M, 256).
     // (a float8 V's byte offsets are half those of the two-byte check)
     for_each_kernel([&](const KernelEntry& e) {
-        const bool q_loader = uses_q_buffer(e.d, e.bn, e.nw, e.causal != 0, e.mode);  // Q through LDS
-        if (st == RSFA_OK && e.dtype == a->dtype && e.d == a->head_dim &&
-            (!loader_offsets_fit(e, a->k_stride[2]) || !loader_offsets_fit(e, a->v_stride[2]) ||
-             (q_loader && !loader_offsets_fit(e, a->q_stride[2]))))
+        if (st == RSFA_OK && e.kg == 1 && e.dtype == a->dtype && e.d == a->head_dim && !loaders_fit(e, a))
             st = RSFA_E_ALIGN;
     });
     if (st != RSFA_OK) return st;
@@ -513,7 +639,7 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
     // hint (RSFA_FLAG_TILE_HINT) or no request the tile the search picks.
     const KernelEntry* e = nullptr;
     if ((st = launch_tile(a, num_cus, &e)) != RSFA_OK) return st;
-    const int bm = e->bm;
+    const int bm = e->rows;
 
     FwdParams p{};
     p.q = a->q;
