@@ -57,16 +57,6 @@ const KernelEntry* find_kernel(int dtype, int d, int bn, int bm, int causal, int
     return hit;
 }
 
-// Whether a tile has key-split variants.
-bool has_keysplit(const KernelEntry& tile) {
-    bool hit = false;
-    for_each_kernel([&](const KernelEntry& e) {
-        if (e.kg > 1 && e.dtype == tile.dtype && e.d == tile.d && e.causal == tile.causal && e.bm == tile.bm && e.bn == tile.bn)
-            hit = true;
-    });
-    return hit;
-}
-
 bool valid_head_dim(int64_t d) { return d == 16 || d == 32 || d == 64 || d == 128 || d == 256; }
 bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
@@ -430,6 +420,7 @@ int validate_request(int causal, int req_bm, int req_bn) {
 int resolve_exact(int64_t d, int causal, int dtype, int req_bm, int req_bn, const KernelEntry** out) {
     const int st = validate_request(causal, req_bm, req_bn);
     if (st != RSFA_OK) return st;
+    if ((*out = find_kernel(dtype, (int)d, req_bn, req_bm, causal, MODE_FUSED)) != nullptr) return RSFA_OK;
     const KernelEntry* best = nullptr;
     double best_dist = 0.0;
     for_each_kernel([&](const KernelEntry& e) {
@@ -579,7 +570,7 @@ static int launch_tile(const rsfa_fwd_args* a, int num_cus, const KernelEntry** 
     int st;
     if (requested) {
         if ((st = resolve_exact(a->head_dim, causal, a->dtype, a->block_m, a->block_n, e)) != RSFA_OK) return st;
-        if (split || !has_keysplit(**e)) return RSFA_OK;
+        if (split) return RSFA_OK;
     }
     const KernelEntry* best = nullptr;
     if ((st = choose_tiling_kept(a->z, a->h, a->n_ctx, a->head_dim, causal, a->dtype, num_cus, &best)) != RSFA_OK)
