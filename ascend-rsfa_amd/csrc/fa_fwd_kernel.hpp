@@ -645,19 +645,21 @@ fa_fwd_kernel(FwdParams p) {
     const Queue qu = make_queue<PAIRS>(p);
     uint32_t* const ctr = p.ticket ? p.ticket + 16 * qu.x : nullptr;
     // A workgroup's first ticket is its rank, and the queue's counter hands out
-    // the tickets from nwg on.  (Drawn like the others, the first one opened
-    // every launch with the round trip of a device-scope atomic, about 4k
-    // cycles: B=2 H=8 S=1024 D=128 causal 29.1 -> 27.7 us, B=1 H=8 S=8192 172.7
-    // -> 170.2, B=32 H=8 S=2048 D=32 230 -> 223.)  Except where pairs run in
-    // lockstep rounds and no task loads the next one's Q early: started in one
-    // burst those workgroups miss L2 on the same tiles together (B=4 H=16 S=8192
-    // D=64 566 us drawn, 570 by rank; B=64 H=8 S=1024 D=256 364 and 367; at
-    // D = 128, B=128 H=8 S=2048, 1241 and 1236).
+    // the tickets from nwg on.  Drawn like the others, the first one opened every
+    // launch with the round trip of a device-scope atomic, about 4k cycles (B=2
+    // H=8 S=1024 D=128 causal 29.1 -> 27.7 us), and went out in order of arrival:
+    // a CU whose workgroups arrived together took several of the heaviest single
+    // blocks, while ranks, dispatched one to a CU first, spread them (B=6 H=6
+    // causal: S=6348 D=16 191 -> 144 us, S=3000 D=64 78.7 -> 70.6, S=3000 D=256
+    // 228 -> 206).  Except where pairs run in lockstep rounds and no task loads
+    // the next one's Q early: started in one burst those workgroups miss L2 on the
+    // same tiles together (B=4 H=16 S=8192 D=64 566 us drawn, 570 by rank; B=64
+    // H=8 S=1024 D=256 364 and 367; at D = 128, B=128 H=8 S=2048, 1241 and 1236).
     constexpr bool DRAW_FIRST = PAIRS && D != 128;
-    const int base = DRAW_FIRST ? 0 : qu.nwg;
+    const int base = DRAW_FIRST && qu.pph ? 0 : qu.nwg;
     int t = task_of_ticket(qu, qu.rank);
     if constexpr (DRAW_FIRST) {
-        if (ctr) {
+        if (ctr && qu.pph) {
             if (tid == 0) *tslot = (int)atomicAdd(ctr, 1u);
             __syncthreads();
             t = task_of_ticket(qu, *tslot);

@@ -673,14 +673,20 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
         const KernelEntry* k = modes[li] == MODE_FUSED ? e
                                : find_kernel(a->dtype, (int)a->head_dim, e->bn, e->bm, causal ? 1 : 0, modes[li]);
         if (!k) return RSFA_E_TILE;
-        const int wgs = resident_wgs(ds, *k);
-        int64_t grid = (int64_t)num_cus * wgs;
-        grid = std::min<int64_t>(grid, p.num_tasks);
-        grid = std::max<int64_t>(grid, 1);
-        p.nq = queue_count(p.num_heads, grid);
-        p.pairs = causal && modes[li] == MODE_FUSED && !(a->flags & RSFA_FLAG_SINGLE_BLOCKS)
-                      ? use_pairs(p.num_heads, p.nmb, grid, p.nq)
-                      : 0;
+        int wgs = resident_wgs(ds, *k);
+        int64_t grid = 0;
+        for (;;) {
+            grid = std::max<int64_t>(1, std::min<int64_t>((int64_t)num_cus * wgs, p.num_tasks));
+            p.nq = queue_count(p.num_heads, grid);
+            p.pairs = causal && modes[li] == MODE_FUSED && !(a->flags & RSFA_FLAG_SINGLE_BLOCKS)
+                          ? use_pairs(p.num_heads, p.nmb, grid, p.nq)
+                          : 0;
+            // Pairs of long rows at head dim 32 gain nothing from more than two
+            // workgroups per CU, whose rounds come more staggered (B*H = 64:
+            // S=8192 458 us with two, 484 with four; S=4096 129 and 116).
+            if (!(p.pairs && e->d == 32 && a->n_ctx >= 8192 && wgs > 2)) break;
+            wgs = 2;
+        }
         p.ticket = nullptr;
         if (!(a->flags & RSFA_FLAG_STATIC_SCHEDULE) && queue_needed(p, grid)) {
             if (!tickets_given) {
