@@ -811,26 +811,40 @@ fa_fwd_kernel(FwdParams p) {
         // QPF: direct load q (< NQD) of this wave's rows into the Q buffer, for
         // the BM rows from qsrc on: block 2*wave + q / QSPB, chunk group q % QSPB.
         // Only this wave reads what it loads there (read_q).
-        auto dma_q = [&](const elem* qsrc, int q) {
-            const int bb = q / QSPB, cg = q % QSPB;
+        auto dma_q_at = [&](const elem* src, uint32_t off, int q) {
             // wave-uniform by construction; made explicit for the SGPR operand
-            const uint64_t a = (uint64_t)(uintptr_t)(qsrc + (int64_t)(32 * wave + 16 * bb) * p.q_sm + cg * 32);
+            const uint64_t a = (uint64_t)(uintptr_t)src;
             const uint64_t ua = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) |
                                 (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a);
-            dma16((const void*)(uintptr_t)ua, qlo, smem_addr + NBUF * BUF + (2 * wave + bb) * BLK + cg * 1024);
+            dma16((const void*)(uintptr_t)ua, off, smem_addr + NBUF * BUF + (2 * wave + q / QSPB) * BLK + (q % QSPB) * 1024);
+        };
+        auto dma_q = [&](const elem* qsrc, int q) {
+            dma_q_at(qsrc + (int64_t)(32 * wave + 16 * (q / QSPB)) * p.q_sm + (q % QSPB) * 32, qlo, q);
         };
         // Where this task's Q comes from (QPF): the Q buffer, filled by the
         // previous task (qready) or by loads issued here for a ping-pong task
-        // of a whole query block (q_dma, read after the first phase's load
-        // wait), else global memory.
-        const bool q_dma = QPF && !qready && jpp > j0 && m0 + BM <= n;
+        // (q_dma, read after the first phase's load wait), else global memory.
+        // Partial blocks take the loads too, rows past the sequence re-reading
+        // its last one (B=16 H=16 S=1000 D=128 139.1 -> 136.9 us, D=64 causal 61.2
+        // -> 60.2), but for causal D = 128: the offsets' registers cost its whole
+        // blocks 0.4 % (B=128 H=8 S=2048 1215 us, 1221 with them).
+        constexpr bool QCLAMP = !(CAUSAL && D == 128);
+        const bool q_dma = QPF && !qready && jpp > j0 && (QCLAMP || m0 + BM <= n);
         int t_next = -1;         // QPF, ticket queue: the next ticket, read at the first barrier
         bool qpf_do = false;     // QPF: this task loads the next task's Q into the Q buffer
         const elem* qnext = qg;  // its first row
         if (jpp > j0) {
             load_k(j0);
             if (q_dma)
-                for (int q = 0; q < NQD; ++q) dma_q(qb + (int64_t)m0 * p.q_sm, q);
+                for (int q = 0; q < NQD; ++q) {
+                    if constexpr (!QCLAMP) {
+                        dma_q(qb + (int64_t)m0 * p.q_sm, q);
+                        continue;
+                    }
+                    const int r0 = min(m0 + 32 * wave + 16 * (q / QSPB), n - 1);
+                    const int rr = min(r0 + ld_rib, n - 1) - r0;
+                    dma_q_at(qb + (int64_t)r0 * p.q_sm + (q % QSPB) * 32, (uint32_t)((rr * p.q_sm + ld_chl * 8) * 2), q);
+                }
             load_v(j0);
             if (j0 + 1 < jpp) load_k(j0 + 1);
         } else if (j0 < j1) {
