@@ -556,6 +556,11 @@ static bool loaders_fit(const KernelEntry& e, const rsfa_fwd_args* a) {
            (!q_loader || loader_offsets_fit(e, a->q_stride[2]));
 }
 
+// Kernels that a call whose rows they cannot address leaves for a tile with
+// fewer keys per load: the key-split variants, and the 128-key tiles of head dims
+// 16 and 32 (their rows may lie twice as far apart with 64).
+static bool has_stand_in(const KernelEntry& e) { return e.kg > 1 || (e.d <= 32 && e.bn > 64); }
+
 // The kernel a launch runs: for a request (block_m, block_n), that of the
 // nearest compiled tile, as the reference's BLOCK_M / BLOCK_N select its
 // kernel's tile; under RSFA_FLAG_TILE_HINT (unless RSFA_FLAG_EXACT_TILE) and
@@ -568,16 +573,16 @@ static int launch_tile(const rsfa_fwd_args* a, int num_cus, const KernelEntry** 
     const bool requested = (a->block_m != 0 || a->block_n != 0) && !hint;
     const bool split = causal && (a->flags & RSFA_FLAG_CAUSAL_SPLIT);
     int st;
-    if (requested) {
-        if ((st = resolve_exact(a->head_dim, causal, a->dtype, a->block_m, a->block_n, e)) != RSFA_OK) return st;
-        if (split) return RSFA_OK;
-    }
-    const KernelEntry* best = nullptr;
-    if ((st = choose_tiling_kept(a->z, a->h, a->n_ctx, a->head_dim, causal, a->dtype, num_cus, &best)) != RSFA_OK)
+    if (requested && (st = resolve_exact(a->head_dim, causal, a->dtype, a->block_m, a->block_n, e)) != RSFA_OK)
         return st;
-    if (best->kg > 1 && (split || !loaders_fit(*best, a)))
-        best = find_kernel(a->dtype, (int)a->head_dim, best->bn, best->bm, causal, MODE_FUSED);
-    if (!requested || (best->kg > 1 && best->bm == (*e)->bm && best->bn == (*e)->bn)) *e = best;
+    if (!requested || !split) {
+        const KernelEntry* best = nullptr;
+        if ((st = choose_tiling_kept(a->z, a->h, a->n_ctx, a->head_dim, causal, a->dtype, num_cus, &best)) != RSFA_OK)
+            return st;
+        if (!requested || (best->kg > 1 && best->bm == (*e)->bm && best->bn == (*e)->bn)) *e = best;
+    }
+    if (has_stand_in(**e) && ((split && (*e)->kg > 1) || !loaders_fit(**e, a)))
+        *e = find_kernel(a->dtype, (int)a->head_dim, (*e)->kg > 1 ? (*e)->bn : 64, (*e)->bm, causal, MODE_FUSED);
     return RSFA_OK;
 }
 
@@ -614,7 +619,7 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
     // <= Z*H*N_CTX rounded up to the largest BLOCK_M, 256).
     // (a float8 V's byte offsets are half those of the two-byte check)
     for_each_kernel([&](const KernelEntry& e) {
-        if (st == RSFA_OK && e.kg == 1 && e.dtype == a->dtype && e.d == a->head_dim && !loaders_fit(e, a))
+        if (st == RSFA_OK && !has_stand_in(e) && e.dtype == a->dtype && e.d == a->head_dim && !loaders_fit(e, a))
             st = RSFA_E_ALIGN;
     });
     if (st != RSFA_OK) return st;

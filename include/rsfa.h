@@ -127,7 +127,11 @@ typedef struct rsfa_fwd_args {
                                  selects the tile: the compiled one nearest to
                                  it runs (rsfa_resolve_tiling), unless
                                  RSFA_FLAG_TILE_HINT.  Split mode sizes its
-                                 workspace with the BLOCK_M that runs        */
+                                 workspace with the BLOCK_M that runs.  Where
+                                 the tile search answers a 128-row tile for a
+                                 grid that does not fill the chip, a fused
+                                 launch of it may split each task's keys over
+                                 its wave groups (on 128 or 64 rows)         */
     int32_t     block_n;      /* requested BLOCK_N (see block_m)                */
     uint32_t    flags;        /* RSFA_FLAG_*                                    */
 } rsfa_fwd_args;
