@@ -201,10 +201,10 @@ fa_fwd_keysplit_kernel(FwdParams p) {
         float m_use = -INFINITY;
         float l_sum = 0.0f;
 
-        // Row max and P of one tile, as in fa_fwd_kernel; a masked tile may
-        // leave a row without any key yet.
-        auto softmax = [&](f32x16(&sacc)[NKT], x8(&pk)[NKT][2], auto masked) {
-            constexpr bool MASK = decltype(masked)::value;
+        // Row max and P of one tile, as in fa_fwd_kernel; but any tile may leave
+        // a row without a finite score yet: a group's first one, whose scores may
+        // all be -inf while other groups' keys are not, or a masked one.
+        auto softmax = [&](f32x16(&sacc)[NKT], x8(&pk)[NKT][2]) {
             float mx = sacc[0][0];
 #pragma unroll
             for (int kt = 0; kt < NKT; ++kt)
@@ -224,7 +224,7 @@ fa_fwd_keysplit_kernel(FwdParams p) {
                     for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
                 m_use = m_new;
             }
-            const float msub = (MASK && m_use == -INFINITY) ? 0.0f : m_use;
+            const float msub = m_use == -INFINITY ? 0.0f : m_use;
 #pragma unroll
             for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
@@ -317,7 +317,7 @@ fa_fwd_keysplit_kernel(FwdParams p) {
         for (; s + 1 < nstep; ++s) {
             phase_barrier();  // Y_s
             __builtin_amdgcn_s_setprio(0);
-            softmax(sacc, pk, std::false_type());
+            softmax(sacc, pk);
             if (s + 3 == nstep) set_offsets(kgo, p.k_sn, rlast);
             if (s + 2 == nstep) set_offsets(vgo, p.v_sn, rlast);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // V_s, K_{s+1}
@@ -344,7 +344,7 @@ fa_fwd_keysplit_kernel(FwdParams p) {
                 for (int i = 0; i < 16; ++i)
                     if (kbase + 32 * kt + 8 * (i >> 2) + 4 * hh + (i & 3) > lim) sacc[kt][i] = -INFINITY;
         }
-        softmax(sacc, pk, std::true_type());
+        softmax(sacc, pk);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         phase_barrier();  // its P.V
         __builtin_amdgcn_s_setprio(1);

@@ -79,3 +79,18 @@ def test_nan_stays_in_its_rows(causal):
     o = forward(q, k, v, causal, 0.125)
     seen = torch.isnan(o[0, 0]).any(-1)
     assert seen[bad if causal else 0:].all() and not (causal and seen[:bad].any())
+
+
+@pytest.mark.parametrize("d,heads,tile", SHAPES)
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("lo,hi", [(20, 1024), (64, 128), (40, 900)])
+def test_keys_scored_minus_infinity(d, heads, tile, causal, lo, hi):
+    # keys lo .. hi - 1 score -inf through a channel (Q's last column 1, K's -inf there):
+    # whole tiles of a key group, its first ones too, while other keys score finite
+    n = 1024
+    q, k, v = oracle.make_inputs(1, heads, n, d, seed=lo)
+    q[..., -1], k[..., -1] = 1.0, 0.0
+    k[:, :, lo:hi, -1] = float("-inf")
+    o, lse = forward(q.cuda(), k.cuda(), v.cuda(), causal, d ** -0.5, return_lse=True)
+    assert torch.isfinite(o).all() and torch.isfinite(lse).all()
+    _check(q[:, :2], k[:, :2], v[:, :2], causal, d ** -0.5, o[:, :2], lse[:, :2])
