@@ -806,7 +806,7 @@ fa_fwd_kernel(FwdParams p) {
         int jpp = j0;
         if constexpr (PP) jpp = min(j1, (CAUSAL ? m0 : n) / BN);
         if constexpr (DIAG_PP || DIAG_VM) {
-            jpp = min(j1, n / BN);  // the diagonal tiles too (whole tiles only)
+            if (m0 + BM <= n) jpp = j1;  // the diagonal tiles too (whole tiles only)
         }
         // QPF: direct load q (< NQD) of this wave's rows into the Q buffer, for
         // the BM rows from qsrc on: block 2*wave + q / QSPB, chunk group q % QSPB.
