@@ -651,11 +651,15 @@ fa_fwd_kernel(FwdParams p) {
     // a CU whose workgroups arrived together took several of the heaviest single
     // blocks, while ranks, dispatched one to a CU first, spread them (B=6 H=6
     // causal: S=6348 D=16 191 -> 144 us, S=3000 D=64 78.7 -> 70.6, S=3000 D=256
-    // 228 -> 206).  Except where pairs run in lockstep rounds and no task loads
-    // the next one's Q early: started in one burst those workgroups miss L2 on the
-    // same tiles together (B=4 H=16 S=8192 D=64 566 us drawn, 570 by rank; B=64
-    // H=8 S=1024 D=256 364 and 367; at D = 128, B=128 H=8 S=2048, 1241 and 1236).
-    constexpr bool DRAW_FIRST = PAIRS && D != 128;
+    // 230 -> 208).  Except for pairs up to head dim 64, which run in lockstep
+    // rounds with no task loading the next one's Q early: started in one burst
+    // those workgroups miss L2 on the same tiles together (D=64: B*H = 64 S=8192
+    // 554 us drawn, 558 by rank, B*H = 512 S=512 51.5 and 53.9; D = 16 and 32
+    // within 2 % either way).  At head dim 256 even code that may draw costs: the
+    // causal kernel's tile loops ran 2 to 3 % longer with it, in launches that
+    // draw nothing (B*H = 8 S=6348 246.6 us, 240.1 without; 16 S=4096 174.5,
+    // 170.7; pairs, B=64 H=8 S=1024, 364 and 362).
+    constexpr bool DRAW_FIRST = PAIRS && D <= 64;
     const int base = DRAW_FIRST && qu.pph ? 0 : qu.nwg;
     int t = task_of_ticket(qu, qu.rank);
     if constexpr (DRAW_FIRST) {

@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 # (head dim, tile, workgroups per CU): the 4-wave tiles run two workgroups on a CU
-@pytest.mark.parametrize("d,tile,per_cu", [(128, (256, 64), 1), (64, (256, 128), 1), (128, (128, 64), 2)])
+@pytest.mark.parametrize("d,tile,per_cu", [(128, (256, 64), 1), (64, (256, 128), 1), (256, (256, 32), 1),
+                                           (128, (128, 64), 2)])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("extra", [-8, 0, 8, 3])
 def test_tickets_around_one_per_workgroup(d, tile, per_cu, causal, extra):
