@@ -220,15 +220,15 @@ def _tiling_module():
     return _TILING
 
 
-def _make_plan(q_, k_, v_, o, v8, causal, BM, BN, hint, split, static_schedule, single_blocks):
+def _make_plan(q_, k_, v_, o, v8, causal, BM, BN, hint, exact, split, static_schedule, single_blocks):
     """The launch arguments of a call but its pointers and scale (the bytes of
     rsfa_fwd_args before, between and after them), and the workspace bytes it
     needs; on the current device, which must be the tensors' device."""
     Z, H, N, D = q_.shape
     lib = _native.lib()
-    # The tile is settled here and passed as an exact request, so the
-    # launch runs the same tile the split workspace is sized for, and a
-    # get_tiling answer from a measured cache is honoured.
+    # The tile is settled here and passed as a request, so the launch runs the
+    # same tile the split workspace is sized for, and a get_tiling answer from a
+    # measured cache is honoured.
     if (BM or BN) and not hint:
         bm, bn = resolve_tiling(D, causal, BM, BN, q_.dtype)
     else:
@@ -244,7 +244,7 @@ def _make_plan(q_, k_, v_, o, v8, causal, BM, BN, hint, split, static_schedule, 
     args.causal = 1 if causal else 0
     args.block_m = bm
     args.block_n = bn
-    args.flags = _native.FLAG_EXACT_TILE | (_native.FLAG_STATIC_SCHEDULE if static_schedule else 0) | (
+    args.flags = (_native.FLAG_EXACT_TILE if exact else 0) | (_native.FLAG_STATIC_SCHEDULE if static_schedule else 0) | (
         _native.FLAG_CAUSAL_SPLIT if (split and causal) else 0) | (
         _native.FLAG_SINGLE_BLOCKS if single_blocks else 0)
     nbytes = int(lib.rsfa_v8_workspace_bytes(Z, H, N, D)) if v8 else 0  # 0: the kernels read the bytes
@@ -268,7 +268,9 @@ def forward(q, k, v, causal, sm_scale, BM=0, BN=0, *, return_lse=False, split=Fa
     runs (``resolve_tiling``); ``BM = BN = 0`` runs ``get_tiling``'s tile.
     ``tile_hint=True`` (default: the ``RSFA_TILE_HINT`` environment variable)
     only checks a request and runs ``get_tiling``'s tile; ``exact_tile=True``
-    overrides hint mode.  ``split=True`` (causal only) runs the reference's
+    overrides hint mode and runs the requested tile's own kernel, where a request
+    for ``get_tiling``'s tile may run a key-split variant of it on small grids.
+    ``split=True`` (causal only) runs the reference's
     two-launch prefix/diagonal split, handing (m, l, acc) over in an fp32
     workspace;
     ``static_schedule=True`` replaces the dynamic task queue by the
@@ -279,7 +281,8 @@ def forward(q, k, v, causal, sm_scale, BM=0, BN=0, *, return_lse=False, split=Fa
     the natural-log logsumexp of the scaled scores, fp32 [Z, H, N].
     """
     hint = _hint_mode(tile_hint, exact_tile) if (BM or BN) else False
-    options = (bool(causal), int(BM), int(BN), hint, bool(split), bool(static_schedule), bool(single_blocks))
+    exact = bool(exact_tile and (BM or BN))
+    options = (bool(causal), int(BM), int(BN), hint, exact, bool(split), bool(static_schedule), bool(single_blocks))
     # The launch arguments but the pointers and the scale depend only on the
     # call's shapes, strides, types, devices and options: memoised while no
     # measured tiling cache is active (its answers may change between calls).  A
@@ -314,10 +317,10 @@ def forward(q, k, v, causal, sm_scale, BM=0, BN=0, *, return_lse=False, split=Fa
         plan = _PLANS.get(key) if memo else None
         if plan is None:
             if q.device.index == torch.cuda.current_device():
-                plan = _make_plan(q_, k_, v_, o, v8, causal, BM, BN, hint, split, static_schedule, single_blocks)
+                plan = _make_plan(q_, k_, v_, o, v8, causal, BM, BN, hint, exact, split, static_schedule, single_blocks)
             else:
                 with torch.cuda.device(q.device):
-                    plan = _make_plan(q_, k_, v_, o, v8, causal, BM, BN, hint, split, static_schedule, single_blocks)
+                    plan = _make_plan(q_, k_, v_, o, v8, causal, BM, BN, hint, exact, split, static_schedule, single_blocks)
             if memo:
                 if len(_PLANS) > 4096:
                     _PLANS.clear()

@@ -169,13 +169,20 @@ def search_case(Z, H, N_CTX, HEAD_DIM, causal, dtype=torch.float16, sm_scale=0.5
     """Time and gate every candidate tiling of one shape.
 
     ``attention_fn(q, k, v, causal, sm_scale, BM, BN)`` defaults to this
-    package's ``forward`` with ``exact_tile=True``; ``candidates`` defaults to ``compiled_candidates``.
+    package's ``forward`` for that request, i.e. to what a ``get_tiling`` answer
+    from the cache will run; where that is a key-split variant of the tile (its
+    output differs from ``exact_tile=True``'s), the record's ``exact_ms`` is the
+    plain kernel's time.  ``candidates`` defaults to ``compiled_candidates``.
     Returns the case record (reference layout plus ``gate``)."""
+    exact_fn = None
     if attention_fn is None:
         from .flash_attention_forward import forward
 
         def attention_fn(q, k, v, causal, sm_scale, bm, bn):
-            # each candidate runs its own instantiation, whatever RSFA_TILE_HINT says
+            # each candidate runs its own tile, whatever RSFA_TILE_HINT says
+            return forward(q, k, v, causal, sm_scale, bm, bn, tile_hint=False)
+
+        def exact_fn(q, k, v, causal, sm_scale, bm, bn):
             return forward(q, k, v, causal, sm_scale, bm, bn, exact_tile=True)
     if device is None:
         device = torch.device("cuda", torch.cuda.current_device())
@@ -202,6 +209,9 @@ def search_case(Z, H, N_CTX, HEAD_DIM, causal, dtype=torch.float16, sm_scale=0.5
                 continue
             rec["avg_ms"] = round(_timer_ms(lambda: attention_fn(q, k, v, causal, sm_scale, bm, bn),
                                             warmup, iters, device), 4)
+            if exact_fn is not None and not torch.equal(o, exact_fn(q, k, v, causal, sm_scale, bm, bn)):
+                rec["exact_ms"] = round(_timer_ms(lambda: exact_fn(q, k, v, causal, sm_scale, bm, bn),
+                                                  warmup, iters, device), 4)
         except (RuntimeError, ValueError, AssertionError) as e:
             rec["error"] = f"{type(e).__name__}: {e}"
             failed.append(rec)

@@ -565,17 +565,18 @@ static bool has_stand_in(const KernelEntry& e) { return e.kg > 1 || (e.d <= 32 &
 // nearest compiled tile, as the reference's BLOCK_M / BLOCK_N select its
 // kernel's tile; under RSFA_FLAG_TILE_HINT (unless RSFA_FLAG_EXACT_TILE) and
 // without a request, the tile search's choice for `num_cus` CUs.  Where that
-// choice is a key-split variant, a request for its tile runs it too; split
-// mode, and rows the variant cannot address, run the tile's plain kernel.
+// choice is a key-split variant, a request for its tile runs it too, unless it
+// is exact; exact requests, split mode, and rows the variant cannot address,
+// run the tile's plain kernel.
 static int launch_tile(const rsfa_fwd_args* a, int num_cus, const KernelEntry** e) {
     const int causal = a->causal != 0;
-    const bool hint = (a->flags & RSFA_FLAG_TILE_HINT) && !(a->flags & RSFA_FLAG_EXACT_TILE);
-    const bool requested = (a->block_m != 0 || a->block_n != 0) && !hint;
+    const bool exact = a->flags & RSFA_FLAG_EXACT_TILE;
+    const bool requested = (a->block_m != 0 || a->block_n != 0) && (exact || !(a->flags & RSFA_FLAG_TILE_HINT));
     const bool split = causal && (a->flags & RSFA_FLAG_CAUSAL_SPLIT);
     int st;
     if (requested && (st = resolve_exact(a->head_dim, causal, a->dtype, a->block_m, a->block_n, e)) != RSFA_OK)
         return st;
-    if (!requested || !split) {
+    if (!requested || !(split || exact)) {
         const KernelEntry* best = nullptr;
         if ((st = choose_tiling_kept(a->z, a->h, a->n_ctx, a->head_dim, causal, a->dtype, num_cus, &best)) != RSFA_OK)
             return st;

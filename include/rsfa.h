@@ -87,9 +87,9 @@ typedef enum rsfa_dtype {
                                           through `workspace` (reference
                                           493-541)                              */
 #define RSFA_FLAG_EXACT_TILE      0x4u /* a request (block_m, block_n) runs the
-                                          compiled tile nearest to it: the
-                                          default, kept for callers of ABI
-                                          version 4; overrides TILE_HINT        */
+                                          compiled tile nearest to it, never a
+                                          key-split variant of the tile (see
+                                          block_m); overrides TILE_HINT         */
 #define RSFA_FLAG_TILE_HINT       0x8u /* a valid request is only checked, and
                                           the tile rsfa_get_tiling picks for
                                           the shape runs                        */
@@ -131,7 +131,8 @@ typedef struct rsfa_fwd_args {
                                  the tile search answers a 128-row tile for a
                                  grid that does not fill the chip, a fused
                                  launch of it may split each task's keys over
-                                 its wave groups (on 128 or 64 rows)         */
+                                 its wave groups (on 128 or 64 rows), unless
+                                 RSFA_FLAG_EXACT_TILE                        */
     int32_t     block_n;      /* requested BLOCK_N (see block_m)                */
     uint32_t    flags;        /* RSFA_FLAG_*                                    */
 } rsfa_fwd_args;

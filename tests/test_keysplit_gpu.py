@@ -94,3 +94,18 @@ def test_keys_scored_minus_infinity(d, heads, tile, causal, lo, hi):
     o, lse = forward(q.cuda(), k.cuda(), v.cuda(), causal, d ** -0.5, return_lse=True)
     assert torch.isfinite(o).all() and torch.isfinite(lse).all()
     _check(q[:, :2], k[:, :2], v[:, :2], causal, d ** -0.5, o[:, :2], lse[:, :2])
+
+
+@pytest.mark.parametrize("d,heads,tile", SHAPES)
+@pytest.mark.parametrize("causal", [False, True])
+def test_exact_tile_runs_the_plain_kernel(d, heads, tile, causal):
+    # kept plans of one shape, with and without exact_tile, stay apart
+    q, k, v = (t.cuda() for t in oracle.make_inputs(1, heads, 1024, d, seed=11))
+    split = forward(q, k, v, causal, d ** -0.5, *tile)
+    exact = forward(q, k, v, causal, d ** -0.5, *tile, exact_tile=True)
+    assert torch.equal(forward(q, k, v, causal, d ** -0.5, *tile), split)
+    assert torch.equal(forward(q, k, v, causal, d ** -0.5), split)
+    assert not torch.equal(exact, split)  # another order of summation
+    want = oracle.reference_attention(q[:, -2:].cpu(), k[:, -2:].cpu(), v[:, -2:].cpu(), causal, d ** -0.5)
+    for o in (exact, split):
+        assert torch.allclose(o[:, -2:].float().cpu(), want, atol=1e-2, rtol=1e-2)
