@@ -675,6 +675,7 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
 
     const int modes[2] = {split ? MODE_PREFIX : MODE_FUSED, MODE_DIAG};
     const int launches = split ? 2 : 1;
+    bool cleared = false;
     for (int li = 0; li < launches; ++li) {
         const KernelEntry* k = modes[li] == MODE_FUSED ? e
                                : find_kernel(a->dtype, (int)a->head_dim, e->bn, e->bm, causal ? 1 : 0, modes[li]);
@@ -699,12 +700,13 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
                 if (dynamic_schedule_allowed(stream)) p.ticket = stream_ticket(ds, stream);
             } else {
                 p.ticket = tickets;
-                if (li == 0) {
-                    // caller-placed counters start each call at zero (a launch
-                    // leaves them at zero, but the caller's buffer may hold
-                    // anything)
+                if (!cleared) {
+                    // caller-placed counters start at zero in the first launch
+                    // of a call that takes them (a launch leaves them at zero,
+                    // but the caller's buffer may hold anything)
                     hipLaunchKernelGGL(clear_words, dim3(1), dim3(64), 0, (hipStream_t)stream, tickets, kSlotWords);
                     if (hipGetLastError() != hipSuccess) return RSFA_E_LAUNCH;
+                    cleared = true;
                 }
             }
         }

@@ -28,3 +28,22 @@ def test_exact_requests_run_the_plain_kernel(tmp_path, entry):
             assert x.params == none.params
         for x in (exact, exact_hint):
             assert x.kernel == "fa" and x.params == {"d": d, "bn": 64, "nw": 4, "causal": causal, "mode": 0}
+
+
+# a split call whose prefix launch has a workgroup per task and whose diagonal launch has not,
+# and the other way round, and neither
+@pytest.mark.parametrize("prefix,diag", [(2, 1), (1, 2), (1, 1)])
+@pytest.mark.parametrize("d", [16, 64])
+def test_callers_counters_are_cleared_before_their_first_use(tmp_path, prefix, diag, d):
+    call = dict(heads=160, n=200, d=d, causal=1, entry="rsfa_attention_fwd_noalloc",
+                flags=_native.FLAG_CAUSAL_SPLIT, block_m=128, block_n=64)  # 320 tasks
+    # (part of the kernel's mangled name: causal, mode)
+    ((st, launches),) = record([call], tmp_path, [("Lb1ELi1E", prefix), ("Lb1ELi2E", diag)])
+    assert st == _native.OK
+    runs = [x for x in launches if x.kernel == "fa"]
+    assert [x.params["mode"] for x in runs] == [1, 2]
+    assert [x.counters for x in runs] == ["scratch" if 320 > 256 * w else "none" for w in (prefix, diag)]
+    first = next(i for i, x in enumerate(launches) if x.kernel == "fa" and x.counters == "scratch")
+    assert [x.kernel for x in launches[:first]].count("clear") == 1
+    assert [x.kernel for x in launches].count("clear") == 1
+    assert all(x.counters == "scratch" for x in launches if x.kernel == "clear")
