@@ -584,7 +584,7 @@ static int launch_tile(const rsfa_fwd_args* a, int num_cus, const KernelEntry** 
     }
     if (has_stand_in(**e) && ((split && (*e)->kg > 1) || !loaders_fit(**e, a)))
         *e = find_kernel(a->dtype, (int)a->head_dim, (*e)->kg > 1 ? (*e)->bn : 64, (*e)->bm, causal, MODE_FUSED);
-    return RSFA_OK;
+    return *e ? RSFA_OK : RSFA_E_TILE;  // (null: a build without the tile that stands in)
 }
 
 // Shared body of the launch entry points.  `ws` / `ws_bytes` is the

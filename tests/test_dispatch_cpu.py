@@ -47,3 +47,24 @@ def test_callers_counters_are_cleared_before_their_first_use(tmp_path, prefix, d
     assert [x.kernel for x in launches[:first]].count("clear") == 1
     assert [x.kernel for x in launches].count("clear") == 1
     assert all(x.counters == "scratch" for x in launches if x.kernel == "clear")
+
+
+def test_rows_past_a_kernels_reach_run_its_stand_in(tmp_path):
+    far = 16909320   # past a 128-key tile's 32-bit offsets, within a 64-key tile's
+    wide = 34087048  # past a 64-key tile's too: for Q at head dim 32 only the key-split loader's
+    calls, want = [], []
+    for d in (16, 32):
+        near = dict(heads=64, n=2048, d=d, dtype=_native.DTYPE_F16)
+        calls += [near, dict(near, k_stride=[0, 0, far, 1]), dict(near, v_stride=[0, 0, far, 1]),
+                  dict(near, block_m=128, block_n=128, k_stride=[0, 0, far, 1]),
+                  dict(near, block_m=128, block_n=128, v_stride=[0, 0, far, 1], flags=_native.FLAG_EXACT_TILE)]
+        want += [("fa", 128)] + 4 * [("fa", 64)]
+    for causal in (0, 1):
+        split = dict(heads=1, n=385, d=32, causal=causal)
+        calls += [split, dict(split, q_stride=[0, 0, wide, 1]),
+                  dict(split, q_stride=[0, 0, wide, 1], block_m=128, block_n=64)]
+        want += [("keysplit", 64), ("fa", 64), ("fa", 64)]
+    got = record(calls, tmp_path)
+    assert [(st, [x.kernel for x in launches]) for st, launches in got] == [(_native.OK, [k]) for k, _ in want]
+    keys = [launches[0].params.get("bn", launches[0].params.get("keys")) for _, launches in got]
+    assert keys == [k for _, k in want]
