@@ -35,8 +35,8 @@ def _parse(line):
 
 def record(calls, tmp_path, occupancy=()):
     """Runs ``calls`` in turn: dicts of rsfa_fwd_args fields, with ``heads``, ``n``
-    and ``d`` for contiguous tensors and optionally ``entry``, ``capturing`` and
-    ``tiling`` (block_m, block_n from rsfa_get_tiling).  ``occupancy``: (part of a
+    and ``d`` for contiguous tensors and optionally ``entry``, ``capturing``,
+    ``stream`` and ``tiling`` (block_m, block_n from rsfa_get_tiling).  ``occupancy``: (part of a
     kernel's mangled name, workgroups per CU).  Returns [(status, [Launch])]."""
     so = os.path.join(str(tmp_path), "librecorder.so")
     if not os.path.exists(so):
@@ -67,6 +67,7 @@ def _child():
         heads, n, d = call.pop("heads"), call.pop("n"), call.pop("d")
         entry = call.pop("entry", "rsfa_attention_fwd")
         rec.recorder_capturing(int(call.pop("capturing", 0)))
+        stream = call.pop("stream", None)
         a = native.FwdArgs()
         a.struct_size = ctypes.sizeof(a)
         a.q = a.k = a.v = a.o = a.workspace = 0x1000
@@ -85,7 +86,7 @@ def _child():
             assert lib.rsfa_get_tiling(1, heads, n, d, a.causal, a.dtype, ctypes.byref(bm), ctypes.byref(bn)) == 0
             a.block_m, a.block_n = bm.value, bn.value
         rec.recorder_clear()
-        st = getattr(lib, entry)(ctypes.byref(a), None)
+        st = getattr(lib, entry)(ctypes.byref(a), ctypes.c_void_p(stream))
         results.append((st, rec.recorder_lines().decode().splitlines()))
     print(json.dumps(results))
 

@@ -2,6 +2,9 @@
 (tests/launch_recorder.py)."""
 import pytest
 
+import test_parity_gpu
+import test_streams_gpu
+import test_zz_no_alloc
 from ascend_rsfa import _native
 from launch_recorder import record
 
@@ -68,3 +71,32 @@ def test_rows_past_a_kernels_reach_run_its_stand_in(tmp_path):
     assert [(st, [x.kernel for x in launches]) for st, launches in got] == [(_native.OK, [k]) for k, _ in want]
     keys = [launches[0].params.get("bn", launches[0].params.get("keys")) for _, launches in got]
     assert keys == [k for _, k in want]
+
+
+# at least the workgroups that fit a CU: one of 8 waves, as many of 4 as a SIMD holds waves of the smallest tiles
+FULL = [("Li8ELb", 1), ("Li4ELb", 4), ("keysplit", 1)]
+
+
+def _queued_calls():
+    for z, h, n, d in test_parity_gpu.QUEUED + test_streams_gpu.QUEUED:
+        for causal in (0, 1):
+            yield dict(heads=z * h, n=n, d=d, causal=causal)
+    codes = {"v8": _native.DTYPE_F16_V8E5M2, "torch.float16": _native.DTYPE_F16, "torch.bfloat16": _native.DTYPE_BF16}
+    for (z, h, n, d), _, causal, dtype, flags in test_zz_no_alloc.QUEUED_CASES:
+        yield dict(heads=z * h, n=n, d=d, causal=int(causal), flags=flags, dtype=codes[str(dtype)])
+
+
+def test_queued_shapes_take_counters_and_captured_streams_none(tmp_path):
+    calls = [dict(c, entry=e, capturing=cap, stream=stream) for c in _queued_calls()
+             for e in ("rsfa_attention_fwd", "rsfa_attention_fwd_noalloc")
+             for cap, stream in ((0, None), (1, None), (0, 2))]  # 2: hipStreamPerThread
+    for call, (st, launches) in zip(calls, record([dict(c) for c in calls], tmp_path, FULL)):
+        assert st == _native.OK, call
+        runs = [x for x in launches if x.kernel != "clear"]
+        assert len(runs) == (2 if call.get("flags") else 1)
+        if call["entry"] == "rsfa_attention_fwd_noalloc":
+            want = "scratch"  # the call's own counters: under capture too
+            assert launches[0].kernel == "clear" and len(launches) == len(runs) + 1
+        else:
+            want = "none" if call["capturing"] or call["stream"] else "allocated"
+        assert {x.counters for x in runs} == {want}, call

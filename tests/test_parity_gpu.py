@@ -317,9 +317,15 @@ def test_nan_inputs_propagate_by_row(causal, D, tile):
         _assert_close(out[0, 1, :512], ref[0, 1, :512], f"D={D} tile={tile} causal head 1 rows < 512")
 
 
+# Shapes with more tasks than workgroups, whose launches take the queue's
+# counters (test_dispatch_cpu.py checks that).
+QUEUED = [(5, 8, 2049, 128), (10, 8, 2049, 64), (6, 8, 1793, 256), (40, 8, 513, 32)]
+
+
+@pytest.mark.parametrize("shape", [(4, 8, 1024, 128)] + QUEUED)
 @pytest.mark.parametrize("causal", [False, True])
-def test_dynamic_and_static_schedules_bitwise_equal(causal):
-    q, k, v = A.make_inputs(4, 8, 1024, 128, seed=15)
+def test_dynamic_and_static_schedules_bitwise_equal(causal, shape):
+    q, k, v = A.make_inputs(*shape, seed=15)
     qd, kd, vd = _to_gpu(q, k, v)
     a = F.forward(qd, kd, vd, causal, 0.09)
     b = F.forward(qd, kd, vd, causal, 0.09, static_schedule=True)
@@ -387,10 +393,11 @@ def test_causal_two_launch_split_matches_fused(BM, BN):
     assert (fused.float() - split.float()).abs().max().item() <= 2.0 ** -10
 
 
-def test_many_launches_across_streams():
-    q, k, v = A.make_inputs(2, 4, 512, 64, seed=17)
+@pytest.mark.parametrize("shape", [(2, 4, 512, 64)] + QUEUED)
+def test_many_launches_across_streams(shape):
+    q, k, v = A.make_inputs(*shape, seed=17)
     qd, kd, vd = _to_gpu(q, k, v)
-    base = F.forward(qd, kd, vd, False, 0.2)
+    base = F.forward(qd, kd, vd, False, 0.2, static_schedule=True)
     torch.cuda.synchronize()
     streams = [torch.cuda.Stream() for _ in range(3)]
     outs = []

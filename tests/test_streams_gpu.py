@@ -6,7 +6,9 @@ stream running its launches in order.  A launch recorded into a HIP graph may
 later be replayed on any stream, concurrently with replays of other graphs
 captured on the same stream, and hipStreamPerThread is one handle for every
 thread's stream; those launches run the static schedule, which gives bitwise
-the results of the dynamic one.  Each replay is checked against the eager
+the results of the dynamic one.  The shapes of QUEUED have more tasks than
+workgroups (test_dispatch_cpu.py checks that): others take no counter at all.
+Each replay is checked against the eager
 result, with eager work and synchronisations between replays.
 """
 import ctypes
@@ -20,10 +22,13 @@ from oracle import attention as A
 
 pytestmark = pytest.mark.gpu
 
+QUEUED = [(5, 8, 2049, 128), (10, 8, 2049, 64)]
 
+
+@pytest.mark.parametrize("shape", [(2, 8, 1024, 128)] + QUEUED)
 @pytest.mark.parametrize("causal", [False, True])
-def test_graphs_replayed_concurrently_on_two_streams(causal):
-    inputs = [[t.cuda() for t in A.make_inputs(2, 8, 1024, 128, seed=s)] for s in (91, 92)]
+def test_graphs_replayed_concurrently_on_two_streams(causal, shape):
+    inputs = [[t.cuda() for t in A.make_inputs(*shape, seed=s)] for s in (91, 92)]
     eager = [F.forward(q, k, v, causal, 0.3) for q, k, v in inputs]
     torch.cuda.synchronize()
     # warm up on a side stream before capture, as torch's graph docs ask
@@ -61,8 +66,9 @@ def test_graphs_replayed_concurrently_on_two_streams(causal):
         assert torch.equal(again, eager[rep % 2])
 
 
-def test_per_thread_default_stream():
-    q, k, v = (t.cuda() for t in A.make_inputs(2, 8, 1024, 128, seed=93))
+@pytest.mark.parametrize("shape", [(2, 8, 1024, 128)] + QUEUED)
+def test_per_thread_default_stream(shape):
+    q, k, v = (t.cuda() for t in A.make_inputs(*shape, seed=93))
     eager = F.forward(q, k, v, True, 0.3)
     o = torch.full_like(q, float("nan"))
     a = _native.FwdArgs()

@@ -4,7 +4,9 @@ It runs the kernels of rsfa_attention_fwd with its queue counters and
 workspace in the library's fixed per-device buffer, so its results must be
 bitwise those of rsfa_attention_fwd on the same arguments.  Each case makes
 two calls in a row on the same buffer, the second on a smaller problem, and
-one case replays the call from a HIP graph.  The size check runs before any
+one case replays the call from a HIP graph.  Launches with a workgroup per task
+take no counters, so some cases have more tasks than workgroups (QUEUED_CASES,
+which test_dispatch_cpu.py checks).  The size check runs before any
 device work and is tested without a GPU.
 """
 import ctypes
@@ -95,10 +97,18 @@ CASES = [
     ((1, 4, 1024, 128), (1, 2, 512, 128), True, "v8", _native.FLAG_CAUSAL_SPLIT),
     ((2, 8, 1024, 128), (1, 3, 500, 128), True, torch.float16, _native.FLAG_STATIC_SCHEDULE),
 ]
+# the same, with more tasks than workgroups in the first shape
+QUEUED_CASES = [
+    ((5, 8, 2049, 128), (1, 4, 300, 128), False, torch.float16, 0),
+    ((5, 8, 2049, 128), (5, 8, 1793, 128), True, torch.bfloat16, 0),
+    ((64, 8, 512, 64), (1, 4, 300, 64), True, torch.float16, 0),  # in pairs
+    ((12, 8, 2049, 16), (2, 4, 513, 16), True, torch.float16, _native.FLAG_CAUSAL_SPLIT),
+    ((12, 8, 2049, 16), (2, 4, 513, 16), True, "v8", _native.FLAG_CAUSAL_SPLIT),
+]
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("big,small,causal,dtype,flags", CASES)
+@pytest.mark.parametrize("big,small,causal,dtype,flags", CASES + QUEUED_CASES)
 def test_noalloc_matches_the_allocating_entry_point_twice_in_a_row(big, small, causal, dtype, flags):
     if dtype == "v8" and _F8 is None:
         pytest.skip("torch has no float8_e5m2")
@@ -107,9 +117,9 @@ def test_noalloc_matches_the_allocating_entry_point_twice_in_a_row(big, small, c
 
 
 @pytest.mark.gpu
-def test_noalloc_under_graph_capture():
+@pytest.mark.parametrize("shape", [(2, 8, 1024, 128), QUEUED_CASES[0][0]])
+def test_noalloc_under_graph_capture(shape):
     lib = _native.lib()
-    shape = (2, 8, 1024, 128)
     q, k, v = (t.cuda() for t in A.make_inputs(*shape, seed=310))
     (o_ref, l_ref, _), _ = _pair(shape, True, 0.3, torch.float16, 0, seed=310)
     o = torch.empty_like(q)
