@@ -86,16 +86,18 @@ int hipStreamIsCapturing(void*, int* status) {
     *status = capturing;
     return 0;
 }
-// One line per launch: kernel, workgroups, threads, then where the counters it
-// gets lie.  clear_words takes their address first, the attention kernels take a
-// struct by value whose last word it is.
+// One line per launch: kernel, workgroups, threads, whether blocks go in pairs, and
+// where the counters it gets lie.  clear_words takes their address first, the
+// attention kernels take a struct by value that holds both.
 int hipLaunchKernel(const void* fn, Dim3 grid, Dim3 block, void** args, size_t, void*) {
     const std::string name = kernels.count(fn) ? kernels[fn] : "?";
     uint64_t ticket;
-    const size_t at = name.find("clear_words") != std::string::npos ? 0 : RECORDER_TICKET_OFFSET;
-    memcpy(&ticket, (const char*)args[0] + at, sizeof(ticket));
+    int32_t pairs = 0;
+    const bool clear = name.find("clear_words") != std::string::npos;
+    memcpy(&ticket, (const char*)args[0] + (clear ? 0 : RECORDER_TICKET_OFFSET), sizeof(ticket));
+    if (!clear) memcpy(&pairs, (const char*)args[0] + RECORDER_PAIRS_OFFSET, sizeof(pairs));
     char tail[96];
-    snprintf(tail, sizeof(tail), " %u %u %s\n", grid.x, block.x, area(ticket));
+    snprintf(tail, sizeof(tail), " %u %u %d %s\n", grid.x, block.x, pairs, area(ticket));
     lines += name + tail;
     return 0;
 }

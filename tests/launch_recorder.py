@@ -15,14 +15,15 @@ _TESTS = os.path.dirname(os.path.abspath(__file__))
 _PKG = os.path.join(os.path.dirname(_TESTS), "ascend-rsfa_amd", "ascend_rsfa")
 
 # kernel: "fa" (d, bn, nw, causal, mode), "keysplit" (d, keys, groups, causal) or "clear"
-Launch = collections.namedtuple("Launch", "kernel params grid threads counters")
+Launch = collections.namedtuple("Launch", "kernel params grid threads pairs counters")
 
-# FwdParams: 7 pointers, 12 strides, 7 ints, c, neg, (4 bytes up to) the counters
-_TICKET_OFFSET = 7 * 8 + 12 * 8 + 9 * 4 + 4
+# FwdParams: 7 pointers, 12 strides, 7 ints (the last: pairs), c, neg, (4 bytes up to) the counters
+_PAIRS_OFFSET = 7 * 8 + 12 * 8 + 6 * 4
+_TICKET_OFFSET = _PAIRS_OFFSET + 3 * 4 + 4
 
 
 def _parse(line):
-    name, grid, threads, counters = line.rsplit(" ", 3)
+    name, grid, threads, pairs, counters = line.rsplit(" ", 4)
     nums = [int(x) for x in re.findall(r"L[ib](\d+)E", name)]
     if "clear_words" in name:
         kind, params = "clear", {}
@@ -30,7 +31,7 @@ def _parse(line):
         kind, params = "keysplit", dict(zip(("d", "keys", "groups", "causal"), nums))
     else:
         kind, params = "fa", dict(zip(("d", "bn", "nw", "causal", "mode"), nums))
-    return Launch(kind, params, int(grid), int(threads), counters)
+    return Launch(kind, params, int(grid), int(threads), int(pairs), counters)
 
 
 def record(calls, tmp_path, occupancy=()):
@@ -41,7 +42,7 @@ def record(calls, tmp_path, occupancy=()):
     so = os.path.join(str(tmp_path), "librecorder.so")
     if not os.path.exists(so):
         subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", f"-DRECORDER_TICKET_OFFSET={_TICKET_OFFSET}",
-                        "-o", so, os.path.join(_TESTS, "launch_recorder.cpp")], check=True)
+                        f"-DRECORDER_PAIRS_OFFSET={_PAIRS_OFFSET}", "-o", so, os.path.join(_TESTS, "launch_recorder.cpp")], check=True)
     spec = json.dumps({"so": so, "pkg": _PKG, "calls": list(calls), "occupancy": list(occupancy)})
     out = subprocess.run([sys.executable, os.path.abspath(__file__)], input=spec, text=True, capture_output=True,
                          timeout=120)

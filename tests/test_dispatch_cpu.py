@@ -2,6 +2,7 @@
 (tests/launch_recorder.py)."""
 import pytest
 
+import test_keysplit_gpu
 import test_parity_gpu
 import test_streams_gpu
 import test_zz_no_alloc
@@ -100,3 +101,15 @@ def test_queued_shapes_take_counters_and_captured_streams_none(tmp_path):
         else:
             want = "none" if call["capturing"] or call["stream"] else "allocated"
         assert {x.counters for x in runs} == {want}, call
+
+
+def test_keysplit_cases_run_the_groups_they_name(tmp_path):
+    cases = test_keysplit_gpu.CASES
+    calls = [dict(heads=h, n=n, d=d, causal=int(c), **tile) for d, _, c, n, h in cases
+             for tile in ({}, {"block_m": 128, "block_n": 64})]
+    got = record(calls, tmp_path, FULL)
+    for (st, launches), case in zip(got, [c for c in cases for _ in range(2)]):
+        (x,) = [x for x in launches if x.kernel != "clear"]
+        assert st == _native.OK and x.kernel == "keysplit" and x.params["groups"] == case[1], case
+        assert not (case in test_keysplit_gpu.PAIRS) or x.pairs, case
+    assert any(x.counters != "none" for _, launches in got for x in launches)  # some of them queued

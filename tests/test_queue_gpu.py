@@ -19,8 +19,8 @@ def test_tickets_around_one_per_workgroup(d, tile, per_cu, causal, extra):
     heads = get_num_compute_cores() * per_cu // 2 + extra  # two query blocks per head
     n = tile[0] + 24
     q, k, v = (t.cuda() for t in oracle.make_inputs(1, heads, n, d, seed=7 + extra))
-    want = forward(q, k, v, causal, 0.125, *tile, static_schedule=True)
+    want = forward(q, k, v, causal, 0.125, *tile, exact_tile=True, static_schedule=True)
     for _ in range(3):
-        assert torch.equal(forward(q, k, v, causal, 0.125, *tile), want)
+        assert torch.equal(forward(q, k, v, causal, 0.125, *tile, exact_tile=True), want)
     ref = oracle.reference_attention(q[:, -2:].cpu(), k[:, -2:].cpu(), v[:, -2:].cpu(), causal, 0.125)
     assert torch.allclose(want[:, -2:].float().cpu(), ref, atol=1e-2, rtol=1e-2)
