@@ -688,10 +688,15 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
             p.pairs = causal && modes[li] == MODE_FUSED && !(a->flags & RSFA_FLAG_SINGLE_BLOCKS)
                           ? use_pairs(p.num_heads, p.nmb, grid, p.nq)
                           : 0;
-            // Pairs of long rows at head dim 32 gain nothing from more than two
-            // workgroups per CU, whose rounds come more staggered (B*H = 64:
-            // S=8192 458 us with two, 484 with four; S=4096 129 and 116).
-            if (!(p.pairs && e->d == 32 && a->n_ctx >= 8192 && wgs > 2)) break;
+            // Long pairs at head dim 32 in exactly two rounds of four workgroups per
+            // CU come too staggered in the second: two per CU (B*H = 128 S=4096
+            // 253 -> 240 us, 64 S=8192 462 -> 448, 32 S=16384 930 -> 878, 16
+            // S=32768 1587 -> 1697).  Not shorter ones (256 S=2048 137 and 152),
+            // nor another number of rounds: one (32 S=8192 226 and 281), three
+            // (96 S=8192 673 and 704), four (128 S=8192 844 and 963); nor a float8 V
+            // (64 S=8192 446 and 479).
+            const int64_t pairs_per_queue = (int64_t)((p.num_heads + p.nq - 1) / p.nq) * (p.nmb / 2);
+            if (!(p.pairs && e->d == 32 && !v8 && a->n_ctx >= 4096 && wgs > 2 && pairs_per_queue == 2 * (grid / p.nq))) break;
             wgs = 2;
         }
         p.ticket = nullptr;

@@ -113,3 +113,14 @@ def test_keysplit_cases_run_the_groups_they_name(tmp_path):
         assert st == _native.OK and x.kernel == "keysplit" and x.params["groups"] == case[1], case
         assert not (case in test_keysplit_gpu.PAIRS) or x.pairs, case
     assert any(x.counters != "none" for _, launches in got for x in launches)  # some of them queued
+
+
+def test_two_workgroups_per_cu_for_long_pairs_in_two_rounds_only(tmp_path):
+    # head dim 32, four workgroups per CU: (heads, keys, workgroups)
+    cases = [(32, 8192, 1024), (64, 8192, 512), (96, 8192, 1024), (128, 8192, 1024), (128, 4096, 512), (64, 4096, 1024),
+             (256, 2048, 1024), (32, 16384, 512)]
+    dtypes = (_native.DTYPE_F16, _native.DTYPE_BF16, _native.DTYPE_F16_V8E5M2)
+    got = record([dict(heads=h, n=n, d=32, causal=1, dtype=dt) for h, n, _ in cases for dt in dtypes], tmp_path, FULL)
+    for (st, (x,)), (h, n, grid, dt) in zip(got, [c + (dt,) for c in cases for dt in dtypes]):
+        assert st == _native.OK and x.pairs == 1 and x.params["nw"] == 4
+        assert x.grid == (1024 if dt == _native.DTYPE_F16_V8E5M2 else grid), (h, n, dt)
