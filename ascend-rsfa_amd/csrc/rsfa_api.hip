@@ -182,11 +182,22 @@ int32_t use_pairs(int64_t num_heads, int32_t nmb, int64_t grid, int32_t nq) {
 // serves its rank in its queue without drawing).  Where every queue has a
 // workgroup per ticket, the counters are left out: the atomic that draws a
 // ticket past the end is then no part of a task (one 64-key tile on 8 heads
-// 5.7 -> 5.5 us, four 197-key ones on 128 heads 10.0 -> 9.4).
-bool queue_needed(const FwdParams& p, int64_t grid) {
+// 5.7 -> 5.5 us, four 197-key ones on 128 heads 10.0 -> 9.4).  Nor where equal
+// tasks (`equal`: non-causal) go to three or more workgroups per CU (`wgs`) in at
+// most two rounds, or in three of which the last is half full or more: drawn, the
+// tasks of a last round that is not full gather on the CUs that ask first, where
+// three share what one could have, while strided by rank they spread over all.
+// Head dim 32, drawn and strided: B*H = 20 S=8192 (1.7 rounds) 330 and 259 us,
+// 256 S=777 (1.75) 48.6 and 41.2, 32 S=8192 (2.7) 442 and 412; head dim 16, 36
+// S=4096 (1.5) 135 and 107.  Otherwise the queue evens out what the rounds drift
+// apart by: 36 S=6348 (2.3) 306 and 317, 1024 S=333 (3) 36.6 and 39.2, 40 S=8192
+// (3.3) 491 and 509.
+bool queue_needed(const FwdParams& p, int64_t grid, bool equal, int wgs) {
     const int64_t heads = (p.num_heads + p.nq - 1) / p.nq;  // of the fullest queue
     const int64_t tickets = heads * (p.pairs ? (p.nmb + 1) / 2 : p.nmb);
-    return tickets > grid / p.nq;
+    const int64_t slots = grid / p.nq;
+    if (equal && wgs >= 3 && (tickets <= 2 * slots || (2 * tickets >= 5 * slots && tickets < 3 * slots))) return false;
+    return tickets > slots;
 }
 
 // Position of an instantiation in the kernel lists (a fixed-size cache index).
@@ -700,7 +711,7 @@ static int fwd_launch(const rsfa_fwd_args* a, void* stream, void* ws, uint64_t w
             wgs = 2;
         }
         p.ticket = nullptr;
-        if (!(a->flags & RSFA_FLAG_STATIC_SCHEDULE) && queue_needed(p, grid)) {
+        if (!(a->flags & RSFA_FLAG_STATIC_SCHEDULE) && queue_needed(p, grid, !causal, wgs)) {
             if (!tickets_given) {
                 if (dynamic_schedule_allowed(stream)) p.ticket = stream_ticket(ds, stream);
             } else {

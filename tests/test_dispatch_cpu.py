@@ -124,3 +124,14 @@ def test_two_workgroups_per_cu_for_long_pairs_in_two_rounds_only(tmp_path):
     for (st, (x,)), (h, n, grid, dt) in zip(got, [c + (dt,) for c in cases for dt in dtypes]):
         assert st == _native.OK and x.pairs == 1 and x.params["nw"] == 4
         assert x.grid == (1024 if dt == _native.DTYPE_F16_V8E5M2 else grid), (h, n, dt)
+
+
+def test_few_rounds_of_equal_tasks_take_no_counters(tmp_path):
+    # (head dim, heads, keys, causal, takes counters), three or four workgroups per CU at head dims 16 and 32
+    cases = [(32, 20, 8192, 0, False), (16, 32, 8192, 0, False), (32, 36, 6348, 0, True), (32, 40, 8192, 0, True),
+             (32, 24, 8192, 0, False), (32, 256, 777, 0, False), (32, 512, 777, 0, True), (16, 1024, 333, 0, True),
+             (32, 20, 16384, 1, True), (64, 20, 8192, 0, True)]
+    got = record([dict(heads=h, n=n, d=d, causal=c) for d, h, n, c, _ in cases], tmp_path,
+                 [("Li64ELi4ELb", 4), ("Li128ELi4ELb", 3)])
+    for (st, (x,)), case in zip(got, cases):
+        assert st == _native.OK and (x.counters != "none") == case[4], case

@@ -319,7 +319,7 @@ def test_nan_inputs_propagate_by_row(causal, D, tile):
 
 # Shapes with more tasks than workgroups, whose launches take the queue's
 # counters (test_dispatch_cpu.py checks that).
-QUEUED = [(5, 8, 2049, 128), (10, 8, 2049, 64), (6, 8, 1793, 256), (40, 8, 513, 32)]
+QUEUED = [(5, 8, 2049, 128), (10, 8, 2049, 64), (6, 8, 1793, 256), (100, 8, 513, 32)]
 
 
 @pytest.mark.parametrize("shape", [(4, 8, 1024, 128)] + QUEUED)
