@@ -829,9 +829,9 @@ fa_fwd_kernel(FwdParams p) {
         // previous task (qready) or by loads issued here for a ping-pong task
         // (q_dma, read after the first phase's load wait), else global memory.
         // Partial blocks take the loads too, rows past the sequence re-reading
-        // its last one (B=16 H=16 S=1000 D=128 139.1 -> 136.9 us, D=64 causal 61.2
-        // -> 60.2), but for causal D = 128: the offsets' registers cost its whole
-        // blocks 0.4 % (B=128 H=8 S=2048 1215 us, 1221 with them).
+        // its last one (B=16 H=16 S=1000 D=128 145.3 -> 142.5 us, B=8 H=16 S=1531
+        // D=64 causal 65.4 -> 64.2), but for causal D = 128: the offsets' registers
+        // cost its whole blocks 0.4 % (B=128 H=8 S=2048 1215 us, 1221 with them).
         constexpr bool QCLAMP = !(CAUSAL && D == 128);
         const bool q_dma = QPF && !qready && jpp > j0 && (QCLAMP || m0 + BM <= n);
         int t_next = -1;         // QPF, ticket queue: the next ticket, read at the first barrier

@@ -19,7 +19,7 @@
 //   B=1 H=8 S=8192 D=128 causal     173.9 -> 132.7 (128 rows, two groups)
 //   B=1 H=32 S=2048 D=128 causal     53.4 -> 43.1
 //   B=5 H=4 S=832 D=64 causal        16.3 -> 12.5 (four)
-//   B=1 H=16 S=4096 D=64 causal      58.6 -> 50.1 (two)
+//   B=1 H=16 S=4096 D=64 causal      57.9 -> 47.8 (two; the rule keeps whole blocks there)
 //   B=2 H=8 S=2048 D=32 causal       26.5 -> 18.7 (four)
 // A two-group step of 128 keys takes the cycles of two 64-key steps of the
 // 256-row kernel on half the rows, about 3.0k; a task's start, merge and store

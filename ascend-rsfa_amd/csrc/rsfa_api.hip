@@ -211,7 +211,7 @@ int kernel_index(const KernelEntry& e) {
 }
 
 // Resident workgroups per CU of an instantiation, queried once per device
-// (a fixed array, so launches allocate no host memory either).
+// (a fixed array: no host memory is allocated for it).
 int resident_wgs(DeviceState& ds, const KernelEntry& e) {
     const int idx = kernel_index(e);
     if (idx >= 0 && idx < kMaxKernels) {
@@ -308,10 +308,13 @@ TileCost tile_cost(const KernelEntry& e, int64_t z, int64_t h, int64_t n, int nu
 // longest task, no less than its work spread over the workgroups, and, filled,
 // no less than 1.5 times that, since the board then runs at its power limit
 // (1.3 times for causal launches at head dim 128, whose short tasks leave the
-// matrix cores idle more: B*H = 32, S=2048 50 us in 256-row blocks, 43 split).
-// Fitted to kernel times of 593 shapes (2 to 256 heads, 64 to 8192 keys, fp16):
-// rms 7 to 10 % (head dim 32: 16 %).  (Head dim 256 has no variant: 128 rows
-// of its Q do not fit the buffers that are free at a task's start.)
+// matrix cores idle more; between the two 32 of 573 choices differ, where 1.3
+// is up to 1.30 times as fast, B*H = 16, S=4096, and down to 0.82, B*H = 40,
+// S=512, in the mean of all 0.1 %).  Against the times of 3372 shapes (1 to 256
+// heads, 64 to 8192 keys, fp16; part of them in
+// profiles/fa_fwd_keysplit_choice.csv) it is off by 10 to 13 % rms.  (Head dim
+// 256 has no variant: 128 rows of its Q do not fit the buffers that are free at
+// a task's start.)
 // ---------------------------------------------------------------------------
 struct LaunchCost {
     int d, rows, bn, kg;  // rows and keys per step of a workgroup
@@ -355,9 +358,10 @@ double launch_us(const KernelEntry& e, int64_t heads, int64_t n, int num_cus) {
 }
 
 // The key-split variant that runs `base`'s shape at least a tenth shorter than
-// `base` (head dim 32, whose predictions are looser: 15 %), or `base`.  Over the
-// fitted shapes 268 run one, 1.15 to 1.22 times as fast in the geometric mean of
-// all; one is slower (B*H = 16, S=4096, D=32: 60.2 -> 63.9 us).
+// `base` (head dim 32, whose predictions are looser: 15 %), or `base`.  Of the
+// 3372 shapes 1371 run one, 1.41 to 1.60 times as fast as `base` in the geometric
+// mean by head dim and mask; 17 of them are slower, by up to a tenth (B*H = 32,
+// S=1200, D=32 causal 16.6 -> 18.3 us).  Always the fastest would be 1 to 4 % more.
 const KernelEntry* keysplit_or(const KernelEntry* base, int64_t heads, int64_t n, int num_cus) {
     const KernelEntry* best = base;
     // (0 without an entry: no variant is shorter)
@@ -392,8 +396,12 @@ int choose_tiling(int64_t z, int64_t h, int64_t n, int64_t d, int causal, int dt
     return RSFA_OK;
 }
 
-// choose_tiling's answer for a launch, kept per thread for the shapes last
-// asked for (the search takes longer than the rest of a launch).
+// choose_tiling's answer for a launch, kept per thread for the shapes last asked
+// for: the search takes 1.7 us, as long as the rest of a launch's checks.  (The C
+// library allocates the table, 2.5 KB, at a thread's first launch.  A table shared
+// by all threads, behind a mutex or sequence numbers, left attention() at 13.9 us
+// instead of 12.5: this library's own thread-local access brings the thread's
+// table of such storage up to date, and other libraries' accesses stay fast.)
 int choose_tiling_kept(int64_t z, int64_t h, int64_t n, int64_t d, int causal, int dtype, int num_cus,
                        const KernelEntry** out) {
     struct Kept {

@@ -154,8 +154,9 @@ int rsfa_attention_fwd(const rsfa_fwd_args *args, void *stream);
  * buffer per device, a static device array of RSFA_NOALLOC_WORKSPACE_BYTES
  * + 4 KiB that the device holds until the process ends.  Problems that need
  * more workspace fail with RSFA_E_SCRATCH before any device work.  The first
- * call on a device looks the buffer up (hipGetSymbolAddress); every call
- * clears its counters with a small kernel on `stream` first.  All calls on one
+ * call on a device looks the buffer up (hipGetSymbolAddress); a call with more
+ * tasks than workgroups clears its counters with a small kernel on `stream`
+ * before the launch that takes them.  All calls on one
  * device share the buffer: calls that overlap in time on one device (other
  * streams, concurrent graph replays) race and must be serialised by the
  * caller. */
