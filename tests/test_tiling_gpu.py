@@ -43,6 +43,8 @@ def test_a_corrupted_tiling_is_rejected_and_cannot_win():
 def test_search_winner_drives_get_tiling():
     print("search Z=2 H=8 N=1024 D=128 causal, then get_tiling from the cache", flush=True)
     rec = tiling.search_case(2, 8, 1024, 128, True, torch.float16, 0.5, warmup=1, iters=3)
+    # the one tile whose request runs a key-split variant also has its plain kernel timed
+    assert [(r["BM"], r["BN"]) for r in rec["all_tested"] if "exact_ms" in r] == [(128, 64)]
     cache = tiling.TilingCache(device_name=torch.cuda.get_device_name())
     cache.add_results({"x": rec})
     best = (rec["best"]["BM"], rec["best"]["BN"])
